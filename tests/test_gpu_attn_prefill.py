@@ -213,3 +213,50 @@ def test_attn_prefill_c3_prompt(env, D):
     for i in (0, 1, 31, 32, 63, 500, 1023, 1024, 1535, 2000, 2015, 2016, 2031):
         want = N.attention(q[i], kc[:i + 1], vc[:i + 1], H_, Hk, a_k, a_v, D)
         assert np.array_equal(got[i].view(np.uint32), want.view(np.uint32)), f"row {i}"
+
+
+# rows of 32-row blocks over caches where the kernel keeps its scores (up to 2048 positions) and where it
+# streams K instead: block remainders, positions at the edges of 32-key tiles and 256-key chunks
+@pytest.mark.parametrize("H_,Hk,hd", [(4, 2, 64), (3, 1, 128)])
+@pytest.mark.parametrize("S,pos,D,ak", [
+    (513, [0, 31, 32, 255, 256, 511, 512], 16, 0.02), (2048, [2047] + list(range(1000, 1032)), 8, 0.02),
+    (2049, [2048], 16, 0.02), (2304, list(range(2238, 2303)), 16, 0.02), (2600, [0, 33, 2303, 2304, 2599], 8, -0.02),
+    (8192, [8191, 5, 8160, 4096], 16, 0.02), (2500, [2499, 7, 300], 16, 0.0), (2500, [2499, 7, 300], 16, np.inf)])
+def test_attn_prefill_long_vs_oracle(env, H_, Hk, hd, S, pos, D, ak):
+    torch, N, ops, T, H = env
+    rng = np.random.default_rng(S + hd + D)
+    kc, vc = caches(rng, S, Hk * hd)
+    pos = np.array(pos, np.int32)
+    q = (rng.standard_normal((len(pos), H_ * hd)) * 2).astype(F)
+    q[-1, 3] = np.inf                                 # head 0 of the last row: its scores are all NaN
+    a_k, a_v = F(ak / np.sqrt(hd)), F(0.03 / 127)
+    print(f"H {H_} hd {hd} S {S} D {D} a_k {a_k}: {len(pos)} rows", flush=True)
+    got = H(ops.attention_prefill(T(q), T(kc), T(vc), T(pos), H_, Hk, a_k, a_v, D))
+    for i in range(0, len(pos), max(1, len(pos) // 7)):
+        p = int(pos[i])
+        with np.errstate(invalid="ignore", over="ignore"):
+            want = N.attention(q[i], kc[:p + 1], vc[:p + 1], H_, Hk, a_k, a_v, D)
+        assert np.array_equal(got[i].view(np.uint32), want.view(np.uint32)), f"row {i} pos {p}"
+
+
+@pytest.mark.parametrize("H_,Hk,hd,S", [(4, 2, 64, 300), (4, 2, 64, 2600), (3, 1, 128, 2100)])
+@pytest.mark.parametrize("qsum,kch,vch", [(True, False, False), (False, True, True), (True, True, True)])
+def test_attn_prefill_options_blocks(env, H_, Hk, hd, S, qsum, kch, vch):
+    """The HF options in the 32-row kernels: 35 rows (a block and a remainder), one of them with a NaN q."""
+    torch, N, ops, T, H = env
+    rng = np.random.default_rng(13 * S + hd)
+    kc, vc = caches(rng, S, Hk * hd)
+    M = 35
+    pos = np.arange(S - M, S, dtype=np.int32)
+    q = (rng.standard_normal((M, H_ * hd)) * 2).astype(F)
+    q[33, 1] = np.nan
+    ch_sk = np.exp(rng.uniform(-4, 1, Hk * hd)).astype(F) * F(0.01) if kch else None
+    ch_av = np.exp(rng.uniform(-3, 2, Hk * hd)).astype(F) * F(1e-3) if vch else None
+    a_k, a_v = F((1.0 if kch else 0.02) / np.sqrt(hd)), F(0.03 / 127)
+    t = lambda a: None if a is None else T(a)
+    got = H(ops.attention_prefill(T(q), T(kc), T(vc), T(pos), H_, Hk, a_k, a_v, 16, qsum, t(ch_sk), t(ch_av)))
+    for i in (0, 1, 31, 32, 33, 34):
+        p = int(pos[i])
+        with np.errstate(invalid="ignore", over="ignore"):
+            want = N.attention(q[i], kc[:p + 1], vc[:p + 1], H_, Hk, a_k, a_v, 16, qsum=qsum, ch_sk=ch_sk, ch_av=ch_av)
+        assert np.array_equal(got[i].view(np.uint32), want.view(np.uint32)), f"row {i} pos {p}"

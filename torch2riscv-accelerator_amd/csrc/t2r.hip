@@ -79,10 +79,15 @@ int ensure_init() {
   for (const void* f : pre)
     if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPreMaxLds) != hipSuccess)
       return T2R_EHIP;
-  if (hipFuncSetAttribute((const void*)k_attn_pw<128, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ap_lds<128>()) != hipSuccess ||
-      hipFuncSetAttribute((const void*)k_attn_pw<64, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ap_lds<64>()) != hipSuccess ||
-      hipFuncSetAttribute((const void*)k_attn_pw<128, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ap_lds<128>()) != hipSuccess ||
-      hipFuncSetAttribute((const void*)k_attn_pw<64, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ap_lds<64>()) != hipSuccess)
+  if (hipFuncSetAttribute((const void*)k_attn_pw<128, 8, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ap_lds<128, 8>()) != hipSuccess ||
+      hipFuncSetAttribute((const void*)k_attn_pw<128, 8, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ap_lds<128, 8>()) != hipSuccess ||
+      hipFuncSetAttribute((const void*)k_attn_pw<64, 8, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ap_lds<64, 8>()) != hipSuccess ||
+      hipFuncSetAttribute((const void*)k_attn_pw<64, 2, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ap_lds<64, 2>()) != hipSuccess)
+    return T2R_EHIP;
+  if (hipFuncSetAttribute((const void*)k_attn_ps<128, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)as_lds<128>()) != hipSuccess ||
+      hipFuncSetAttribute((const void*)k_attn_ps<128, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)as_lds<128>()) != hipSuccess ||
+      hipFuncSetAttribute((const void*)k_attn_ps<64, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)as_lds<64>()) != hipSuccess ||
+      hipFuncSetAttribute((const void*)k_attn_ps<64, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)as_lds<64>()) != hipSuccess)
     return T2R_EHIP;
   // the GEMM's deep-ring configuration: 128 KB of LDS, one workgroup per CU
   const void* deep[] = {(const void*)k_gemm_d<EPI_STORE, false, 128, 4>, (const void*)k_gemm_d<EPI_STORE, true, 128, 4>,
@@ -159,13 +164,16 @@ bool pre_ok(const AttnArgs& a) {
   return a.hd % 16 == 0 && a.hd <= 128 && attn_pre_lds_bytes(pre_cap(a), (a.hd + 31) & ~31) <= kPreMaxLds;
 }
 // ... and its 32-row form (k_attn_pw): head dims 128 and 64 without the HF options, rows attending to at
-// most ap_keys positions
+// most the 2048 positions whose scores a block keeps in registers. Past them, and with the options, the
+// streamed form (ps_takes) is the faster one of what is left: see the kernels for both sides.
 bool pw_ok(const AttnArgs& a) {
   if (attn_opt(a) || !(a.D == 8 || a.D == 16)) return false;
-  return (a.hd == 128 && pre_cap(a) <= ap_keys<128>()) || (a.hd == 64 && pre_cap(a) <= ap_keys<64>());
+  return (a.hd == 128 || a.hd == 64) && pre_cap(a) <= ap_keys<8>();
 }
 // the multi-row ATTN_ONLY launch runs k_attn_pw (only then may q come as int8 rows: AttnArgs::q8)
 inline bool pw_takes(const AttnArgs& a) { return a.tab != nullptr && a.kv_row_stride == 0 && pw_ok(a); }
+
+inline bool ps_takes(const AttnArgs& a) { return a.tab != nullptr && a.kv_row_stride == 0 && (a.hd == 128 || a.hd == 64); }
 
 // batch-1 decode attention split over workgroups per head (k_attn_dec's SPLIT forms): the heads of a
 // model whose shape takes it (head dim 128, caches over 512 rows, 4 splits a head in at most 256
@@ -184,9 +192,8 @@ int attn_launch(int mode, const AttnArgs& a, int rows, hipStream_t st) {
   if (a.H <= 0 || a.Hk <= 0 || a.H % a.Hk || a.hd <= 0 || a.hd > kMaxHd || a.hd % 8 || a.S <= 0 || a.S > kMaxS ||
       (a.D != 8 && a.D != 16))
     return T2R_ESHAPE;
-  // int8 q rows (AttnArgs::q8) pass from the prep kernels at head dims 64 / 128 to k_attn_pw only
-  if (a.q8 != nullptr && (mode == ATTN_FUSED || (mode == ATTN_PREP && a.hd != 64 && a.hd != 128) ||
-                          (mode == ATTN_ONLY && !pw_takes(a))))
+  // int8 q rows (AttnArgs::q8) pass from the prep kernels to k_attn_pw at head dim 128 only
+  if (a.q8 != nullptr && (mode == ATTN_FUSED || a.hd != 128 || (mode == ATTN_ONLY && !pw_takes(a))))
     return T2R_ESHAPE;
   const size_t lds = mode == ATTN_PREP ? 0 : attn_lds_bytes(a.S, a.D);
   dim3 grid(a.H, rows), block(kAttnThreads);
@@ -262,14 +269,23 @@ int attn_launch(int mode, const AttnArgs& a, int rows, hipStream_t st) {
     else launch(k_attn_prep, pg, pb, 0, st, a);
   } else if (pw_takes(a)) {
     const dim3 grid_pw(a.H, cdiv(rows, kApRows));
-    // (q quantized by the prep kernel when the caller set q8: the Q8I form)
-    if (a.q8 != nullptr) {
-      if (a.hd == 128) launch((k_attn_pw<128, true>), grid_pw, dim3(kApThreads), ap_lds<128>(), st, a, rows);
-      else launch((k_attn_pw<64, true>), grid_pw, dim3(kApThreads), ap_lds<64>(), st, a, rows);
-    } else if (a.hd == 128) {
-      launch((k_attn_pw<128, false>), grid_pw, dim3(kApThreads), ap_lds<128>(), st, a, rows);
+    // (q quantized by the prep kernel when the caller set q8: the Q8I form, at head dim 128)
+    if (a.hd == 128) {
+      if (a.q8 != nullptr) launch((k_attn_pw<128, 8, true>), grid_pw, dim3(kApThreads), ap_lds<128, 8>(), st, a, rows);
+      else launch((k_attn_pw<128, 8, false>), grid_pw, dim3(kApThreads), ap_lds<128, 8>(), st, a, rows);
+    } else if (pre_cap(a) <= ap_keys<2>()) {
+      launch((k_attn_pw<64, 2, false>), grid_pw, dim3(kApThreads), ap_lds<64, 2>(), st, a, rows);
     } else {
-      launch((k_attn_pw<64, false>), grid_pw, dim3(kApThreads), ap_lds<64>(), st, a, rows);
+      launch((k_attn_pw<64, 8, false>), grid_pw, dim3(kApThreads), ap_lds<64, 8>(), st, a, rows);
+    }
+  } else if (ps_takes(a)) {
+    const dim3 grid_ps(a.H, cdiv(rows, kApRows));
+    if (a.hd == 128) {
+      if (opt) launch((k_attn_ps<128, true>), grid_ps, dim3(kApThreads), as_lds<128>(), st, a, rows);
+      else launch((k_attn_ps<128, false>), grid_ps, dim3(kApThreads), as_lds<128>(), st, a, rows);
+    } else {
+      if (opt) launch((k_attn_ps<64, true>), grid_ps, dim3(kApThreads), as_lds<64>(), st, a, rows);
+      else launch((k_attn_ps<64, false>), grid_ps, dim3(kApThreads), as_lds<64>(), st, a, rows);
     }
   } else if (a.tab != nullptr && a.kv_row_stride == 0 && pre_ok(a)) {
     const int hdp = (a.hd + 31) & ~31;

@@ -24,6 +24,8 @@
 // (channel c = g hd + j of the cache row). The specialised kernels take them in a separate
 // instantiation (template flag OPT), so the default one is unchanged.
 #pragma once
+#include <limits.h>
+
 #include "t2r_device.h"
 
 namespace t2r {
@@ -82,7 +84,7 @@ struct AttnArgs {
   // the model's status word (nullptr: none): bit 1 a split's bounded wait ran out, bit 2 a row's
   // position was outside the cache (the row is then neither read nor written)
   int32_t* status;
-  // prefill at head dims 64 / 128: the prep kernels' quant_act of each q head vector, the int8 rows
+  // prefill at head dim 128: the prep kernels' quant_act of each q head vector, the int8 rows
   // [rows, q8_stride] and the scales [rows, H], written instead of the fp32 q and read by the
   // 32-row attention (k_attn_pw's Q8I form); nullptr: q stays fp32 in qkv
   int8_t* q8;
@@ -1637,8 +1639,8 @@ inline size_t attn_pre_lds_bytes(int S, int HDP) {
 }
 
 // ------------------------------------------------------------------ prefill attention, 32-row blocks
-// k_attn_pre's numerics without the HF options at head dims 128 (up to 2048 positions) and 64 (up to
-// 512), one 512-thread workgroup per (query head, 32 rows): every K and V byte read serves 32 rows,
+// k_attn_pre's numerics without the HF options at head dims 128 and 64 over up to 2048 positions,
+// one 512-thread workgroup per (query head, 32 rows): every K and V byte read serves 32 rows,
 // and the MFMAs' 32 query columns / rows are all rows of the block. Wave w owns the key tiles (32
 // keys) w, w + 8, ... (TW of them at the largest T) from the scores to P.V, and keeps them in
 // registers:
@@ -1660,19 +1662,22 @@ inline size_t attn_pre_lds_bytes(int S, int HDP) {
 //    read (ds_read_b64_tr_b8), two reads a B operand gathering column n's bytes of the A operand's
 //    keys; HD / 32 MFMAs a tile;
 //  - the waves' int32 sums added by LDS integer atomics (exact in any order) and scaled.
-// HD 128 keeps 8 tiles a wave (128 score registers, one workgroup per CU, a four-tile K ring, two
-// exp-chunk buffers); HD 64 keeps 2 (512 positions), so that two workgroups share a CU.
+// TW 8 (up to 2048 positions) keeps 8 tiles a wave: 128 score registers, one workgroup per CU, a
+// four-tile K ring, two exp-chunk buffers. TW 2 (512 positions, head dim 64) leaves room for two
+// workgroups a CU. Bound by the VALU steps of a key (about 40, 14 of them EXP). 512 rows of 32 heads at
+// head dim 64 attending to 1520..2031 positions: 36.6 us, against 104 in k_attn_pre's 16-row blocks
+// (which read K and V twice as often and run one thread per key chain) and 44.3 streamed (k_attn_ps);
+// at 512..1023 positions 22.8, 61 and 25.6 us.
 constexpr int kApRows = 32, kApThreads = 512, kApWaves = kApThreads / 64;
 constexpr int kApStage = 256 + 16;                       // float stride of a row of a 256-key chunk
-template <int HD> struct ApCfg;
-template <> struct ApCfg<128> { static constexpr int TW = 8, RING = 4, NSB = 2, MINB = 1; };
-template <> struct ApCfg<64> { static constexpr int TW = 2, RING = 2, NSB = 1, MINB = 2; };
-template <int HD> constexpr int ap_keys() { return 32 * kApWaves * ApCfg<HD>::TW; }   // positions a row may attend to
+// TW: the tiles a wave keeps (TW 256 positions)
+template <int HD, int TW> struct ApCfg { static constexpr int RING = TW == 2 ? 2 : 4, NSB = TW == 2 ? 1 : 2, MINB = TW == 2 ? 2 : 1; };
+template <int TW> constexpr int ap_keys() { return 32 * kApWaves * TW; }   // positions a row may attend to
 // dynamic LDS: the waves' K rings, then (reused) the exp-chunk buffers, then (reused) the waves'
 // transposed V tiles
-template <int HD> constexpr size_t ap_lds() {
-  constexpr size_t ring = (size_t)kApWaves * ApCfg<HD>::RING * 32 * HD;
-  constexpr size_t stage = (size_t)ApCfg<HD>::NSB * kApRows * kApStage * 4;
+template <int HD, int TW> constexpr size_t ap_lds() {
+  constexpr size_t ring = (size_t)kApWaves * ApCfg<HD, TW>::RING * 32 * HD;
+  constexpr size_t stage = (size_t)ApCfg<HD, TW>::NSB * kApRows * kApStage * 4;
   constexpr size_t vt = (size_t)kApWaves * HD * 32;
   return ring > stage ? (ring > vt ? ring : vt) : (stage > vt ? stage : vt);
 }
@@ -1688,9 +1693,9 @@ T2R_DEV v2i_t lds_read_tr8(int8_t* p) {
 // block's rows are loaded straight into the score MFMA's B operands, and the SFU tables, the P.V sums'
 // zeroing and the row bounds go to LDS after the scores, before the barrier the row maxima need
 // anyway (no barrier before the scores).
-template <int HD, bool Q8I>
-__global__ __launch_bounds__(kApThreads, ApCfg<HD>::MINB) void k_attn_pw(AttnArgs a, int M) {
-  constexpr int KS = HD / 32, NW = kApWaves, TW = ApCfg<HD>::TW, RING = ApCfg<HD>::RING, NSB = ApCfg<HD>::NSB;
+template <int HD, int TW, bool Q8I>
+__global__ __launch_bounds__(kApThreads, (ApCfg<HD, TW>::MINB)) void k_attn_pw(AttnArgs a, int M) {
+  constexpr int KS = HD / 32, NW = kApWaves, RING = ApCfg<HD, TW>::RING, NSB = ApCfg<HD, TW>::NSB;
   constexpr int CPR = HD / 16;                    // 16-byte chunks of a K row
   constexpr int NDMA = HD / 32;                   // DMA instructions (1 KB) a K tile
   constexpr int TB = 32 * HD;                     // bytes of a K tile
@@ -2064,6 +2069,375 @@ __global__ __launch_bounds__(kApThreads, ApCfg<HD>::MINB) void k_attn_pw(AttnArg
       for (int u = 0; u < CPT / 4; ++u) {
         const v4i_t sv = *(const v4i_t*)&O[m * OST + c0 + 4 * u];
         *(v4f_t*)(out + 4 * u) = v4f_t{(float)sv.x * a.a_v, (float)sv.y * a.a_v, (float)sv.z * a.a_v, (float)sv.w * a.a_v};
+      }
+    }
+  }
+}
+
+// ------------------------------------------------------------------ prefill attention, streamed
+// The same 32-row blocks for rows that attend to any number of positions (up to kMaxS), with or without
+// the HF options: no score is kept. K passes by the block's waves two or three times (from L2: a block's
+// head re-reads what it just read), each pass forming the int8 dot products again on the matrix cores:
+//  1. the row maxima. With a finite a_k != 0 the score F(F(f32(acc) s_q) a_k) is monotone in the int32
+//     acc, so the maximum is the score of the largest acc (the smallest, a_k < 0): one integer
+//     maximum a key instead of the two products;
+//  2. (without qsum) e = EXP(s - max) into LDS, 256 keys at a time, and the D-lane ordered sums, as in
+//     k_attn_pw;
+//  3. e again, p = to_i8(...) packed as the MFMA A operand, P.V, as in k_attn_pw.
+// K and V tiles come by LDS DMA into slots of the wave's own, each refilled as soon as its operands
+// are in registers, and a wave's tiles need no registers beyond the one at hand, so two workgroups
+// share a CU: one's chains and barriers overlap the other's EXPs. Bound by the VALU (two EXPs a key,
+// about 45 steps without qsum). 1001 rows of 32 heads at head dim 64 from position 2500: 127 us, against
+// 1190 in k_attn's workgroup per (head, row); with qsum (one EXP a key, no chains) 777 rows of 16 heads at
+// head dim 128 from position 500: 27.6 us, against 74.4 in k_attn_pre.
+template <int HD> struct AsCfg { static constexpr int RING = HD == 64 ? 2 : 1; };
+template <int HD> constexpr size_t as_lds() {             // K slots, then the exp chunk / the V slots
+  constexpr size_t k = (size_t)kApWaves * AsCfg<HD>::RING * 32 * HD;
+  constexpr size_t stage = (size_t)kApRows * kApStage * 4, v = (size_t)kApWaves * 32 * HD;
+  return k + (stage > v ? stage : v);
+}
+
+template <int HD, bool OPT>
+__global__ __launch_bounds__(kApThreads, 4) void k_attn_ps(AttnArgs a, int M) {
+  constexpr int KS = HD / 32, NW = kApWaves, RING = AsCfg<HD>::RING;
+  constexpr int CPR = HD / 16;                    // 16-byte chunks of a K row
+  constexpr int NDMA = HD / 32;                   // DMA instructions (1 KB) a tile
+  constexpr int TB = 32 * HD;                     // bytes of a tile
+  constexpr int NQ = HD / 64;                     // q elements a lane and row
+  constexpr int NCT = HD / 32;                    // P.V column tiles
+  constexpr int OST = HD + 8;                     // int32 stride of a row of the P.V sums
+  static_assert((size_t)kApRows * OST * 4 <= as_lds<HD>(), "the P.V sums reuse the dynamic LDS");
+  extern __shared__ __align__(16) float big[];
+  __shared__ __align__(16) float tab[kSfuWords];
+  __shared__ __align__(16) float2 et[kSfuExpPairs];
+  __shared__ __align__(16) int8_t Q8[kApRows][HD];
+  __shared__ __align__(16) float s_mx[kApRows][NW];
+  __shared__ float s_sq[kApRows], s_r[kApRows];
+  __shared__ int s_T[kApRows], s_ps[kApRows];
+  const int h = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * kApRows, tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 31, half = lane >> 5;
+  const int G = a.H / a.Hk, g = h / G, S = a.S, D = a.D;
+  const int cap = a.t_cap > 0 && a.t_cap < S ? a.t_cap : S;
+  const int kv_dim = a.Hk * HD;
+  const bool qsum = OPT && a.qsum;
+
+  // ---- the loads that depend on nothing, unconditional (as k_attn_pw)
+  const int pn = a.pos[min(r0 + n, M - 1)];
+  float qx[kApRows / NW][NQ];
+#pragma unroll
+  for (int k = 0; k < kApRows / NW; ++k) {
+    const int r = min(r0 + wave + NW * k, M - 1);
+    const float* q = a.qkv + (long long)r * a.qkv_stride + (long long)h * HD;
+#pragma unroll
+    for (int e = 0; e < NQ; ++e) qx[k][e] = q[lane + 64 * e];
+  }
+  const v4f_t tv = ((const v4f_t*)a.tab)[tid & (kSfuWords / 4 - 1)];      // (stored by tid < kSfuWords / 4)
+  const float2 ev = sfu_exp_pair(min(tid, kSfuExpPairs - 1), a.tab);      // (stored by tid < kSfuExpPairs)
+  if constexpr (OPT) {
+    if (a.ch_sk != nullptr)                       // K per channel: the scales folded into q
+#pragma unroll
+      for (int e = 0; e < NQ; ++e) {
+        const float sk = a.ch_sk[g * HD + lane + 64 * e];
+#pragma unroll
+        for (int k = 0; k < kApRows / NW; ++k) qx[k][e] = qx[k][e] * sk;
+      }
+  }
+  if (tid < kSfuWords / 4) ((v4f_t*)tab)[tid] = tv;   // (before the DMA, whose count the compiler cannot know)
+  if (tid < kSfuExpPairs) et[tid] = ev;
+  const int Tn = r0 + n < M && pn >= 0 && pn < S ? min(pn + 1, cap) : 0;
+  const int ntile = ((int)wave_max_u32((uint32_t)Tn) + 31) / 32;   // lanes n cover the 32 rows
+  const int nown = ntile > wave ? (ntile - wave + NW - 1) / NW : 0;  // tiles this wave owns: wave + 8 j
+  const int Tmin = (int)~wave_max_u32(~(Tn > 0 ? (uint32_t)Tn : 0xFFFFFFFFu));
+
+  // ---- tiles by LDS DMA: whole rows, chunk kc of row r at 16-byte slot CPR r + (kc ^ swz(r)); rows
+  // past the cache are clamped to its last (their keys are past every T)
+  auto swz = [](int r) { return CPR == 8 ? ((r ^ (r >> 3)) & 7) : ((r >> 2) & 3); };
+  int8_t* ring = (int8_t*)big + wave * (RING * TB);
+  float* sb = (float*)((int8_t*)big + NW * RING * TB);
+  int8_t* vt = (int8_t*)sb + wave * TB;
+  // this lane's 16-byte chunk of instruction i, whose row is (64 i + lane) / CPR: swz of it is that of
+  // row lane / CPR, at head dim 128 XOR i
+  const uint32_t col0 = (uint32_t)(g * HD + 16 * ((lane % CPR) ^ swz(lane / CPR)));
+  auto issue = [&](const int8_t* base, int8_t* dst, int j) {
+    const int ti = wave + NW * j;
+#pragma unroll
+    for (int i = 0; i < NDMA; ++i) {
+      const int row = min(32 * ti + (64 * i + lane) / CPR, S - 1);
+      __builtin_amdgcn_global_load_lds((const void*)(base + (long long)row * kv_dim + (col0 ^ (HD == 128 ? 16u * i : 0u))), (void*)(dst + 1024 * i), 16, 0, 0);
+    }
+  };
+  auto k_issue = [&](int j) { issue(a.kc, ring + TB * (j % RING), j); };
+  auto k_start = [&]() {
+#pragma unroll
+    for (int j = 0; j < RING; ++j)
+      if (j < nown) k_issue(j);
+  };
+  auto wait_vm = [&](int groups) {                 // at most `groups` tiles' requests outstanding
+    if (groups >= 2) __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * NDMA));
+    else if (groups == 1) __builtin_amdgcn_s_waitcnt(waitcnt_vm(NDMA));
+    else __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+    asm volatile("" ::: "memory");
+  };
+  k_start();
+
+  // ---- q of the block's rows to int8 (k_attn_pw's steps); invalid rows 0
+  if (wave == 0 && half == 0) {
+    s_T[n] = Tn;
+    s_ps[n] = 0;
+  }
+  lds_barrier();
+  {
+    uint32_t am[kApRows / NW];
+#pragma unroll
+    for (int k = 0; k < kApRows / NW; ++k) {
+      uint32_t m = abs_bits(qx[k][0]);
+#pragma unroll
+      for (int e = 1; e < NQ; ++e) m = max(m, abs_bits(qx[k][e]));
+      am[k] = wave_max_u32(m);
+    }
+    static_assert(kApRows / NW == 4, "four rows a wave");
+    const uint32_t mine = lane == 0 ? am[0] : lane == 1 ? am[1] : lane == 2 ? am[2] : am[3];
+    const float sq_l = fv(mine) * kInv127;
+    const float inv_l = sfu_recip(sq_l, tab);
+#pragma unroll
+    for (int k = 0; k < kApRows / NW; ++k) {
+      const int i = wave + NW * k;
+      const bool ok = __shfl(Tn, i) > 0;            // lane i holds row i
+      const float inv = ok ? fv((uint32_t)__builtin_amdgcn_readlane((int)fb(inv_l), k)) : 0.0f;
+#pragma unroll
+      for (int e = 0; e < NQ; ++e) Q8[i][lane + 64 * e] = (int8_t)to_i8(qx[k][e] * inv);
+      if (lane == k) s_sq[i] = sq_l;
+    }
+  }
+  lds_barrier();
+  const float sqn = s_sq[n];
+  v4i_t qb[KS];                                      // (head dim 128: read again for each tile, for the registers)
+  auto q_read = [&]() {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qb[ks] = *(const v4i_t*)&Q8[n][32 * ks + 16 * half];
+  };
+  if constexpr (HD == 64) q_read();
+
+  // ---- tile j's dot products: wait for its DMA (groups: requests issued after it that may be in
+  // flight), its A fragments to registers, the slot refilled with tile j + RING, KS MFMAs. Lane
+  // (n, half) gets row n's keys 32 ti + 8 (r / 4) + 4 half + r % 4.
+  auto dots = [&](int j, int groups) {
+    wait_vm(groups);
+    const int8_t* kt = ring + TB * (j % RING);
+    v4i_t ka[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) ka[ks] = *(const v4i_t*)(kt + 16 * (CPR * n + ((2 * ks + half) ^ swz(n))));
+    __builtin_amdgcn_s_waitcnt(0xc07f);              // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    if (j + RING < nown) k_issue(j + RING);
+    if constexpr (HD == 128) q_read();
+    v16i_t acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(ka[ks], qb[ks], acc, 0, 0, 0);
+    return acc;
+  };
+  const int koff = 4 * half;
+  auto key = [&](int ti, int r) { return 32 * ti + 8 * (r >> 2) + koff + (r & 3); };
+
+  // ---- pass 1: the row maxima
+  float rmx = -__builtin_inff();
+  if (__builtin_isfinite(a.a_k) && a.a_k != 0.0f) {
+    const int flip = a.a_k < 0.0f ? -1 : 0;          // the largest ~acc is the smallest acc
+    int im = INT_MIN;
+    for (int j = 0; j < nown; ++j) {
+      const v16i_t acc = dots(j, min(nown - 1 - j, RING - 1));
+      const int ti = wave + NW * j;
+      if (32 * ti + 32 <= Tmin) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) im = max(im, acc[r] ^ flip);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) im = max(im, key(ti, r) < Tn ? acc[r] ^ flip : INT_MIN);
+      }
+    }
+    if (im != INT_MIN) rmx = ((float)(im ^ flip) * sqn) * a.a_k;   // (|acc| <= 127^2 HD: no acc is INT_MIN)
+  } else {
+    for (int j = 0; j < nown; ++j) {
+      const v16i_t acc = dots(j, min(nown - 1 - j, RING - 1));
+      const int ti = wave + NW * j;
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (key(ti, r) < Tn) rmx = smax(rmx, ((float)acc[r] * sqn) * a.a_k);
+    }
+  }
+  k_start();                                         // the next pass's first tiles
+  rmx = smax(rmx, __shfl_xor(rmx, 32));
+  if (half == 0) s_mx[n][wave] = rmx;
+  lds_barrier();
+  float mx;
+  {
+    const v4f_t m0 = *(const v4f_t*)&s_mx[n][0], m1 = *(const v4f_t*)&s_mx[n][4];
+    mx = smax(smax(smax(m0.x, m0.y), smax(m0.z, m0.w)), smax(smax(m1.x, m1.y), smax(m1.z, m1.w)));
+  }
+  // every valid row's maximum finite: y in [0, 127] and to_i8(y) is y's RNE integer (k_attn_pw)
+  const bool fast = __all(Tn == 0 || __builtin_isfinite(mx));
+  // e of the lane's key r of tile ti from its dot product, keys past T +0 (mask: the tile may hold some)
+  auto exp1 = [&](int acc, int ti, int r, bool mask) {
+    const float x = sfu_exp_sm(((float)acc * sqn) * a.a_k - mx, et);
+    return mask && key(ti, r) >= Tn ? 0.0f : x;
+  };
+
+  // ---- pass 2: the D-lane ordered sums (k_attn_pw's chunks: chunk k is tile 8 k + w of wave w)
+  if (!qsum) {
+    const int cpr = 64 / D, cr = wave * cpr + lane / D, cl = lane % D;
+    const bool chain = cr < kApRows;
+    const int nchunk = (ntile + NW - 1) / NW;
+    const int sx = (n >> 2) & 3, cx = (cr >> 2) & 3;
+    const int wb0 = n * kApStage + 4 * ((8 * wave + half) ^ sx), wb1 = n * kApStage + 4 * ((8 * wave + 2 + half) ^ sx);
+    const int cb0 = cr * kApStage + 4 * ((cl >> 2) ^ cx) + (cl & 3);
+    const int cb1 = cr * kApStage + 4 * ((2 + (cl >> 2)) ^ cx) + (cl & 3);      // D 8: odd u
+    float acc = 0.0f;
+    for (int k = 0; k < nchunk; ++k) {
+      float e[16];
+      if (k < nown) {
+        const v16i_t ac = dots(k, min(nown - 1 - k, RING - 1));
+        const int ti = wave + NW * k;
+        if (32 * ti + 32 <= Tmin) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) e[r] = exp1(ac[r], ti, r, false);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) e[r] = exp1(ac[r], ti, r, true);
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) e[r] = 0.0f;
+      }
+      if (k > 0) lds_barrier();                      // the previous chunk's chain reads come first
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr)
+        *(v4f_t*)(sb + ((rr & 1) ? wb1 : wb0) + 16 * (rr >> 1)) = v4f_t{e[4 * rr], e[4 * rr + 1], e[4 * rr + 2], e[4 * rr + 3]};
+      lds_barrier();
+      if (chain) {
+        if (D == 16) {
+          const float* c0 = sb + cb0;
+          float v[16];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) v[u] = c0[16 * u];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) acc = acc + v[u];
+        } else {
+          const float* c0 = sb + cb0;
+          const float* c1 = sb + cb1;
+#pragma unroll
+          for (int h8 = 0; h8 < 2; ++h8) {
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = (u & 1) ? c1[16 * ((16 * h8 + u) >> 1)] : c0[16 * ((16 * h8 + u) >> 1)];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) acc = acc + v[u];
+          }
+        }
+      }
+    }
+    acc = lane_tree_rows(acc, D, cl);
+    if (chain && cl == 0) s_r[cr] = sfu_recip(acc, tab);
+    k_start();
+    lds_barrier();                                   // s_r, and every chain's reads before the V slots' DMA
+  }
+
+  // ---- pass 3: p and P.V. Lane (column n, half)'s B operand is read back transposed from the V tile
+  // in the K slots' layout (k_attn_pw); V tile j + 1 is requested once tile j's operands are read.
+  uint32_t tr0;                                      // column tile 0's first read in the tile
+  {
+    const int gq = lane >> 4, b = (lane & 15) >> 1, row = 8 * (b >> 2) + 4 * (gq >> 1) + (b & 3);
+    tr0 = (uint32_t)(row * HD + 16 * ((gq & 1) ^ swz(row)) + 8 * (lane & 1));
+  }
+  // column tile c's reads: slot bits 5 and up by XOR (swz(row + 16) = swz(row) ^ 2 at head dim 128, swz(row) at 64)
+  auto tr = [&](int c, int t) {
+    return vt + (tr0 ^ (uint32_t)(32 * c) ^ (t && HD == 128 ? 32u : 0u)) + 16 * HD * t;
+  };
+  const float rn = qsum ? 0.0f : s_r[n];
+  v16i_t pv[NCT];
+#pragma unroll
+  for (int c = 0; c < NCT; ++c)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) pv[c][r] = 0;
+  int psum = 0;
+  if (nown > 0) issue(a.vc, vt, 0);
+  for (int j = 0; j < nown; ++j) {
+    const v16i_t ac = dots(j, min(nown - 1 - j, RING - 1) + 1);
+    const int ti = wave + NW * j;
+    uint32_t w4[4];
+    auto probs = [&](bool mask, auto to_word) {      // four keys at a time: few values live beside the sums
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        float y[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float x = exp1(ac[4 * rr + c], ti, 4 * rr + c, mask);
+          y[c] = (qsum ? x : x * rn) * 127.0f;
+        }
+        w4[rr] = to_word(y);
+        if constexpr (HD == 128) __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // y in [0, 127] (fast): v_cvt_pk_u8_f32 rounds to nearest even and inserts the byte
+    auto cvt = [](const float (&y)[4]) {
+      uint32_t w = 0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) w = __builtin_amdgcn_cvt_pk_u8_f32(y[c], c, w);
+      return w;
+    };
+    if (fast && 32 * ti + 32 <= Tmin) probs(false, cvt);
+    else if (fast) probs(true, cvt);
+    else probs(true, [](const float (&y)[4]) { return (uint32_t)pack_i8x4(to_i8(y[0]), to_i8(y[1]), to_i8(y[2]), to_i8(y[3])); });
+    if constexpr (OPT) {
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) psum = __builtin_amdgcn_sdot4((int)w4[rr], 0x01010101, psum, false);
+    }
+    const v4i_t pa = v4i_t{(int)w4[0], (int)w4[1], (int)w4[2], (int)w4[3]};
+    wait_vm(j + RING < nown ? 1 : 0);                // V tile j (K tile j + RING came after it)
+    v2i_t lo[NCT], hi[NCT];
+#pragma unroll
+    for (int c = 0; c < NCT; ++c) {
+      lo[c] = lds_read_tr8(tr(c, 0));
+      hi[c] = lds_read_tr8(tr(c, 1));
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);              // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    if (j + 1 < nown) issue(a.vc, vt, j + 1);
+#pragma unroll
+    for (int c = 0; c < NCT; ++c)
+      pv[c] = __builtin_amdgcn_mfma_i32_32x32x32_i8(pa, v4i_t{lo[c].x, lo[c].y, hi[c].x, hi[c].y}, pv[c], 0, 0, 0);
+  }
+
+  // ---- the waves' sums (exact int32 atomics), then the scaled output of the valid rows
+  int* O = (int*)big;
+  __syncthreads();                                   // every wave's tile reads before the sums reuse the slots
+  for (int k = tid; k < kApRows * OST; k += kApThreads) O[k] = 0;
+  if constexpr (OPT) {
+    if (qsum && nown > 0) atomicAdd(&s_ps[n], psum);
+  }
+  __syncthreads();
+  if (nown > 0) {
+#pragma unroll
+    for (int c = 0; c < NCT; ++c)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int m = 8 * (r >> 2) + 4 * half + (r & 3);
+        atomicAdd(&O[m * OST + 32 * c + n], pv[c][r]);
+      }
+  }
+  __syncthreads();
+  {
+    constexpr int CPT = HD / 16;                   // output columns a thread
+    const int m = tid >> 4, c0 = CPT * (tid & 15);
+    if (s_T[m] > 0) {
+      float* out = a.att + (long long)(r0 + m) * a.att_stride + (long long)h * HD + c0;
+      const float rq = qsum ? qsum_scale(s_ps[m], tab) : 0.0f;
+#pragma unroll
+      for (int u = 0; u < CPT; ++u) {
+        float y = (float)O[m * OST + c0 + u];
+        if (qsum) y = y * rq;
+        out[u] = y * (OPT && a.ch_av != nullptr ? a.ch_av[g * HD + c0 + u] : a.a_v);
       }
     }
   }
