@@ -339,3 +339,41 @@ def test_shape_errors_raise(env):
         ops.linear(T(np.zeros((4, 24), np.int8)), T(np.ones(4, F)), T(np.zeros(24, np.int8)), T(np.ones(1, F)))
     with pytest.raises(ValueError):
         ops.moe_route(T(np.zeros((1, 70), F)), 4, 16)
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 4095, 4097, 32767, 32768, 32773, 128257])
+def test_argmax_edges(env, n):
+    """Rows of any length and alignment: ties at both ends, signed zeros, a late and an early NaN, all -inf."""
+    torch, N, ops, T, H = env
+    rng = np.random.default_rng(n)
+    x = np.tile((rng.standard_normal(n)).astype(F), (7, 1))
+    x[0, [0, n - 1, n // 2]] = 9.0
+    x[1] = -np.abs(x[1]) - 1
+    x[1, n // 3:] = -0.0
+    x[1, n - 1] = 0.0                                 # equal to the -0.0 before it
+    x[2, n - 1] = np.nan
+    x[3, [n // 2, n - 1]] = np.nan
+    x[4] = -np.inf
+    x[5, n - 1] = np.inf
+    x[6] = np.arange(n)
+    got = H(ops.argmax(T(x)))
+    assert list(got) == [int(np.argmax(r)) for r in x]
+
+
+@pytest.mark.parametrize("rows,n", [(3, 16), (2, 1024), (2, 1040), (3, 2048), (1, 4112), (2, 8192)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_row_ops_alignment(env, rows, n, off):
+    """RMSNorm and quant_act of 16-byte aligned rows (the staged kernels) and of the same rows one float on."""
+    torch, N, ops, T, H = env
+    rng = np.random.default_rng(n + off)
+    flat = np.zeros(rows * n + off, F)
+    flat[off:] = rng.standard_normal(rows * n) * 3
+    x = flat[off:].reshape(rows, n)
+    g = (1 + 0.1 * rng.standard_normal(n)).astype(F)
+    t = T(flat)[off:].view(rows, n)
+    for D in (8, 16):
+        got = H(ops.rmsnorm(t, T(g), 1e-5, D))
+        assert np.array_equal(got.view(np.uint32), N.rmsnorm(x, g, 1e-5, D).view(np.uint32))
+    xq, s = ops.quant_act(t)
+    wq, ws = N.quant_act(x)
+    assert np.array_equal(H(xq), wq) and np.array_equal(H(s).view(np.uint32), ws.view(np.uint32))
