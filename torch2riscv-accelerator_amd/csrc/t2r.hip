@@ -176,14 +176,15 @@ inline bool pw_takes(const AttnArgs& a) { return a.tab != nullptr && a.kv_row_st
 inline bool ps_takes(const AttnArgs& a) { return a.tab != nullptr && a.kv_row_stride == 0 && (a.hd == 128 || a.hd == 64); }
 
 // batch-1 decode attention split over workgroups per head (k_attn_dec's SPLIT forms): the heads of a
-// model whose shape takes it (head dim 128, caches over 512 rows, 4 splits a head in at most 256
-// workgroups), else 0
+// model whose shape takes it (caches of more than one pass of the kernel: 512 rows at head dim 128, 1024
+// at 64; 4 splits a head in at most 256 workgroups), else 0
 constexpr int kSplits = 4;
 inline int split_heads(const t2r_model_desc& d) {
-  return d.head_dim == 128 && d.seq_len > 512 && d.heads * kSplits <= 256 ? d.heads : 0;
+  const bool passes = (d.head_dim == 128 && d.seq_len > 512) || (d.head_dim == 64 && d.seq_len > 2048);
+  return passes && d.heads * kSplits <= 256 ? d.heads : 0;
 }
 inline bool attn_split(const AttnArgs& a, int rows) {
-  return a.nsplit > 1 && rows == 1 && a.hd == 128 && a.sp_s && a.sp_o && a.sp_acc && a.sp_sync;
+  return a.nsplit > 1 && rows == 1 && (a.hd == 128 || a.hd == 64) && a.sp_s && a.sp_o && a.sp_acc && a.sp_sync;
 }
 // ... and whether it leaves its int32 P.V sums per split for the next linear (SPLIT 2) instead of att
 inline bool attn_split_to_linear(const AttnArgs& a, int rows) { return attn_split(a, rows) && !attn_opt(a); }
@@ -233,8 +234,13 @@ int attn_launch(int mode, const AttnArgs& a, int rows, hipStream_t st) {
     if (attn_split(a, rows)) {
       // (without the HF options the next linear adds the splits' sums: attn_split_to_linear)
       const dim3 gs(a.H, a.nsplit);
-      if (opt) launch((k_attn_dec<8, true, 1>), gs, block, dl, st, a);
-      else launch((k_attn_dec<8, false, 2>), gs, block, dl, st, a);
+      if (a.hd == 64) {
+        if (opt) launch((k_attn_dec<4, true, 1>), gs, block, dl, st, a);
+        else launch((k_attn_dec<4, false, 2>), gs, block, dl, st, a);
+      } else {
+        if (opt) launch((k_attn_dec<8, true, 1>), gs, block, dl, st, a);
+        else launch((k_attn_dec<8, false, 2>), gs, block, dl, st, a);
+      }
     } else if (opt) {
       switch (a.hd / 16) {
         case 1: launch((k_attn_dec<1, true>), grid, block, dl, st, a); break;
@@ -336,11 +342,12 @@ struct Model {
   int8_t* mxq;
   float* msx;
   int32_t* status;
-  // batch-1 decode attention split over workgroups per head (nsplit > 1; 0 when the shape does not take
-  // it or the device cannot hold a launch's workgroups at once): published scores [H, S] and SPLIT 2's
+  // batch-1 decode attention split over workgroups per head (nsplit > 1; 0 when the shape or the workspace does
+  // not take it or the device cannot hold a launch's workgroups at once): published scores [H, S] and SPLIT 2's
   // per-split P.V sums [4, H, kMaxHd] (both within one step); SPLIT 1's met sums [H, kMaxHd] and the
   // arrival counters [H, 2], carried from launch to launch (zeroed at creation)
   int nsplit = 0;
+  int hs = 0;                       // heads the workspace holds split state for (0: no split)
   float* sp_s;
   int32_t* sp_o;
   int32_t* sp_acc;
@@ -415,7 +422,7 @@ long long carve(Model* m, char* base, int M, char* state = nullptr, bool ext_sta
   const t2r_model_desc& d = m->d;
   Carve c{base, 0}, cs{state, 0};
   Carve& st = ext_state ? cs : c;
-  const int hs = split_heads(d);
+  const int hs = m->hs;
   m->status = st.take<int32_t>(1);
   m->sp_sync = st.take<uint32_t>(2LL * hs);
   m->sp_acc = st.take<int32_t>((long long)hs * kMaxHd);
@@ -434,8 +441,6 @@ long long carve(Model* m, char* base, int M, char* state = nullptr, bool ext_sta
   m->mxq = c.take<int8_t>((long long)M * d.dim);
   m->msx = c.take<float>(M);
   m->pos_rows = c.take<int32_t>(M);
-  m->sp_s = c.take<float>((long long)hs * d.seq_len);
-  m->sp_o = c.take<int32_t>((long long)kSplits * hs * kMaxHd);
   if (d.n_experts > 0) {
     const long long routes = (long long)M * k;
     m->moe_off = c.take<int32_t>(d.n_experts + 1);
@@ -447,7 +452,12 @@ long long carve(Model* m, char* base, int M, char* state = nullptr, bool ext_sta
   // split-K partial sums of the prefill linears: 4 splits of up to 2048 rows of the widest
   // STORE / RESID output (C3's 2032-row prompt: 133 MB)
   m->part_rows = M < 2048 ? M : 2048;
-  m->part = c.take<int32_t>(4LL * m->part_rows * (m->qkv_dim > d.dim ? m->qkv_dim : d.dim));
+  // ... which a decode step does not use: the split attention's scores and sums are in the same bytes
+  const long long part = 4LL * m->part_rows * (m->qkv_dim > d.dim ? m->qkv_dim : d.dim);
+  const long long sc = ((long long)hs * d.seq_len + 63) / 64 * 64, split = sc + (long long)kSplits * hs * kMaxHd;
+  m->part = c.take<int32_t>(part > split ? part : split);
+  m->sp_s = (float*)m->part;
+  m->sp_o = m->part ? m->part + sc : nullptr;
   return c.off;
 }
 
@@ -461,6 +471,7 @@ void model_dims(Model* m) {
   if (m->q_dim > mi) mi = m->q_dim;
   if (d.hidden > mi) mi = d.hidden;
   m->max_in = mi;
+  m->hs = split_heads(d);
 }
 
 // the caller's descriptor as the current version: an ABI-1 descriptor ends before the HF options,
@@ -652,8 +663,8 @@ AttnArgs layer_attn_args(Model* m, int l, const int32_t* pos, int mode) {
   at.tab = sfu_table_ptr();
   at.qsum = d.attn_qsum;
   at.status = m->status;
-  // batch-1 decode at head dim 128 over caches of more than 512 rows: each head's keys over 4
-  // workgroups (k_attn_dec's SPLIT form), all of them resident at once (checked at creation)
+  // batch-1 decode over caches of more than one pass: each head's keys over 4 workgroups (k_attn_dec's
+  // SPLIT form), all of them resident at once (checked at creation)
   if (mode == RUN_DECODE && m->nsplit > 1) {
     at.nsplit = m->nsplit;
     at.sp_s = m->sp_s; at.sp_o = m->sp_o; at.sp_acc = m->sp_acc; at.sp_sync = m->sp_sync;
@@ -898,7 +909,9 @@ bool split_fits(const t2r_model_desc& d, int heads) {
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return false;
-  const void* ks[] = {(const void*)k_attn_dec<8, false, 2>, (const void*)k_attn_dec<8, true, 1>};
+  const void* k8[] = {(const void*)k_attn_dec<8, false, 2>, (const void*)k_attn_dec<8, true, 1>};
+  const void* k4[] = {(const void*)k_attn_dec<4, false, 2>, (const void*)k_attn_dec<4, true, 1>};
+  const auto& ks = d.head_dim == 64 ? k4 : k8;
   for (const void* k : ks) {
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, kAttnThreads, attn_dec_lds_bytes(d.seq_len, d.D)) !=
@@ -917,10 +930,16 @@ int model_init(Model* m, const t2r_model_desc& dv, char* state = nullptr, long l
   const t2r_model_desc* desc = &m->d;
   model_dims(m);
   long long sb = 0;
-  if (carve(m, nullptr, desc->max_rows, nullptr, state != nullptr, &sb) > desc->workspace_bytes || sb > (state ? state_cap : sb))
-    return T2R_ENOMEM;
+  auto fits = [&]() {
+    return carve(m, nullptr, desc->max_rows, nullptr, state != nullptr, &sb) <= desc->workspace_bytes &&
+           sb <= (state ? state_cap : sb);
+  };
+  if (!fits()) {
+    m->hs = 0;                                       // a workspace that holds all but the split attention's part
+    if (!fits()) return T2R_ENOMEM;
+  }
   carve(m, (char*)desc->workspace, desc->max_rows, state, state != nullptr);
-  const int hs = split_heads(m->d);
+  const int hs = m->hs;
   m->nsplit = hs > 0 && split_fits(m->d, hs) ? kSplits : 0;
   // the carried state starts clear: the status word, the split counters and SPLIT 1's sums
   if (hipMemset(m->status, 0, sizeof(int32_t)) != hipSuccess ||

@@ -26,6 +26,8 @@
 #pragma once
 #include <limits.h>
 
+#include <type_traits>
+
 #include "t2r_device.h"
 
 namespace t2r {
@@ -118,6 +120,11 @@ T2R_DEV void split_wait(uint32_t* p, uint32_t want, int32_t* status) {
   }
   if (status) atomicOr(status, 2);
 }
+
+// The head (or KV head split) of grid column x of n: workgroups go to the eight XCDs in turn, so columns
+// x, x + 8, ... share an XCD and its L2; they take neighbouring heads, whose K / V rows are the same
+// (a KV head's group) or share 128-byte lines (head dim 64).
+T2R_DEV int xcd_col(int x, int n) { return (n & 7) ? x : (x & 7) * (n >> 3) + (x >> 3); }
 
 inline bool attn_opt(const AttnArgs& a) { return a.qsum || a.ch_sk || a.ch_isk || a.ch_isv || a.ch_av; }
 
@@ -447,7 +454,10 @@ T2R_DEV int slot_group_sum(int v) {
 
 // SPLIT (batch-1 decode of long caches): grid y splits a head's keys, workgroup j taking passes
 // j, j + n, ... (n = min(nsplit, passes); the others end at once). One CU streams a head's K and V
-// at most ~95 GB/s (522 KB at head dim 128 and T = 2048), so more CUs per head shorten that part.
+// at most ~95 GB/s (522 KB at head dim 128 and T = 2048; half of it at head dim 64, whose rows are half a
+// 128-byte line), so more CUs per head shorten that part. At head dim 64 n is 1 up to two passes (2048
+// positions): their stream costs less than the exchange (C4's step at 1500 positions 580 us in one
+// workgroup a head, 611 in two), past them it does not (at 6100: 692 us against 780 in one).
 // Each split publishes its scores with device-coherent stores and arrives once; after one bounded
 // wait every split reads all T scores and forms the max, the EXPs, the ordered sum and RECIP itself
 // (the same bits in each), then the probabilities and P.V of its own passes. The splits past the
@@ -456,6 +466,9 @@ T2R_DEV int slot_group_sum(int v) {
 // writes the output and clears the sums and its counter for the next launch. SPLIT 2 (no HF
 // options): each split stores its own int32 sums (splits past the passes store zeros) and the next
 // linear's prologue adds the four and scales them (F(f32(sum) a_v), the output's own formula).
+// C4's decode step at 6100 positions: 844 us with one workgroup a head, its query heads' workgroups on
+// different XCDs and the chain's values read 16 ahead; 692 us split, a KV head's workgroups on one XCD
+// (xcd_col: 780 without) and 32 ahead; at 2000 positions 601 -> 567 us, at 600 518 -> 511.
 template <int NCH, bool OPT = false, int SPLIT = 0>   // 16-byte chunks per head row: hd = 16 NCH; OPT: the HF options
 __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
   constexpr int HD = 16 * NCH;
@@ -469,13 +482,14 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
   __shared__ __align__(16) float tab[kSfuWords];
   __shared__ __align__(16) float s_k[HD], s_q[HD], s_v[HD];
   __shared__ __align__(16) int s_qq[HD / 4], s_kq[HD / 4], s_vq[HD / 4];
-  __shared__ int part[kAttnWaves * 4][HD];
+  __shared__ __align__(16) int part[kAttnWaves * 4][HD];
   __shared__ float red[16];
   __shared__ float s_sq, s_r;
   __shared__ int s_qs[kAttnWaves];
   __shared__ int s_last;
 
-  const int h = blockIdx.x, row = SPLIT ? 0 : blockIdx.y, tid = threadIdx.x;
+  const int h = xcd_col(blockIdx.x, a.H);
+  const int row = SPLIT ? 0 : blockIdx.y, tid = threadIdx.x;
   const int sj = SPLIT ? blockIdx.y : 0;         // this workgroup's split
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // (uniform: scalar selects by wave)
   const int G = a.H / a.Hk, g = h / G, S = a.S;
@@ -527,7 +541,16 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
   const bool pos_ok = pos_in >= 0 && pos_in < S;
   const int pos = pos_ok ? pos_in : 0;
   const int T = pos + 1;
-  const int nsp = SPLIT ? min(a.nsplit, (T + TS * R - 1) / (TS * R)) : 1;   // splits with passes
+  // splits with passes; head dim 64: one up to two passes, whose second costs less than the exchange
+  const int nsp = SPLIT && !(HD == 64 && T <= 2 * TS * R) ? min(a.nsplit, (T + TS * R - 1) / (TS * R)) : 1;
+  // SPLIT: splits past the number of passes end here (all of a launch's workgroups agree on it; SPLIT 2:
+  // with zero sums)
+  if (SPLIT && sj >= nsp) {
+    if (SPLIT == 2)
+      for (int j = tid; j < HD; j += kAttnThreads) a.sp_o[(long long)sj * q_dim + (long long)h * HD + j] = 0;
+    if (tid == 0) __hip_atomic_fetch_add(a.sp_sync + 2 * h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
   const int c = tid & (NCHP - 1), ts = tid / NCHP;
   const bool cok = c < NCH;
   // cache rows [0, pos): byte range of this KV head's columns up to row pos
@@ -620,15 +643,6 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
     }
   }
   __syncthreads();
-  // SPLIT: splits past the number of passes end here (all of a launch's workgroups agree on it; not
-  // before the head vectors' first use, so that no branch lets the compiler sink their loads below
-  // the position's wait); SPLIT 2: with zero sums
-  if (SPLIT && sj >= nsp) {
-    if (SPLIT == 2)
-      for (int j = tid; j < HD; j += kAttnThreads) a.sp_o[(long long)sj * q_dim + (long long)h * HD + j] = 0;
-    if (tid == 0) __hip_atomic_fetch_add(a.sp_sync + 2 * h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return;
-  }
 #pragma unroll
   for (int i = 0; i < R; ++i) vw[i] = buffer_load16(vrs, chunk_off(sj * TS * R + ts + TS * i));
 
@@ -691,38 +705,47 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
       const bool ok = t < T;
       sc[ok ? osum_index(t, D, P) : dummy] = sv;
       mloc = smax(mloc, ok ? sv : -__builtin_inff());
-      if (SPLIT && ok) __hip_atomic_store(a.sp_s + (long long)h * S + t, sv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (SPLIT && nsp > 1 && ok) __hip_atomic_store(a.sp_s + (long long)h * S + t, sv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
   if constexpr (SPLIT) {
     // every split's scores published (every wave's stores complete before the barrier, so thread 0's
     // release covers all of them), then all T of them into sc from the published copy (the own ones
     // read back unchanged); the max over them
-    wave_mem_done();
-    __syncthreads();
+    // (a single split's scores are all its own: it only counts its arrival)
     uint32_t* arrive = a.sp_sync + 2 * h;
-    if (tid == 0) {
-      const uint32_t old = __hip_atomic_fetch_add(arrive, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-      const uint32_t ns = (uint32_t)a.nsplit;
-      split_wait(arrive, old - old % ns + ns, a.status);
-    }
-    __syncthreads();
-    mloc = -__builtin_inff();
-    const float* pub = a.sp_s + (long long)h * S;
-    for (int t0 = 0; t0 < T; t0 += 4 * kAttnThreads) {   // four loads in flight per thread
-      float sv[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        sv[u] = __hip_atomic_load(pub + min(t0 + u * kAttnThreads + tid, T - 1), __ATOMIC_RELAXED,
-                                  __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int t = t0 + u * kAttnThreads + tid;
-        if (t < T) {
-          sc[osum_index(t, D, P)] = sv[u];
-          mloc = smax(mloc, sv[u]);
-        }
+    if (nsp > 1) {
+      wave_mem_done();
+      __syncthreads();
+      if (tid == 0) {
+        const uint32_t old = __hip_atomic_fetch_add(arrive, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t ns = (uint32_t)a.nsplit;
+        split_wait(arrive, old - old % ns + ns, a.status);
       }
+      __syncthreads();
+      mloc = -__builtin_inff();
+      const float* pub = a.sp_s + (long long)h * S;
+      auto gather = [&](auto nu, int t0) {           // nu loads in flight per thread
+        constexpr int NU = decltype(nu)::value;
+        float sv[NU];
+#pragma unroll
+        for (int u = 0; u < NU; ++u)
+          sv[u] = __hip_atomic_load(pub + min(t0 + u * kAttnThreads + tid, T - 1), __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+          const int t = t0 + u * kAttnThreads + tid;
+          if (t < T) {
+            sc[osum_index(t, D, P)] = sv[u];
+            mloc = smax(mloc, sv[u]);
+          }
+        }
+      };
+      int t0 = 0;
+      for (; T - t0 > 4 * kAttnThreads; t0 += 8 * kAttnThreads) gather(std::integral_constant<int, 8>(), t0);
+      if (t0 < T) gather(std::integral_constant<int, 4>(), t0);
+    } else if (tid == 0) {
+      __hip_atomic_fetch_add(arrive, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
   mloc = wave_smax(mloc);
@@ -737,24 +760,35 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
   // lanes the groups g < Tpad / D (row t = g D + d; +0 at t >= T), conflict-free runs of words
   const int Gt = (T + D - 1) / D;
   const bool two = D > kAttnWaves;
-  for (int g0 = 0; g0 < Gt; g0 += 64) {
-    const int gg = g0 + lane;
-    if (gg < Gt) {
-      float* p0 = sc + wave * P + gg;
-      float* p1 = p0 + kAttnWaves * P;
-      const float v0 = *p0, v1 = two ? *p1 : 0.0f;
-      const float e0 = sfu_exp_np(v0 - m, tab);
-      *p0 = gg * D + wave < T ? e0 : 0.0f;
-      if (two) {
-        const float e1 = sfu_exp_np(v1 - m, tab);
-        *p1 = gg * D + wave + kAttnWaves < T ? e1 : 0.0f;
+  // (two runs of 64 groups a step, all their EXPs side by side: the table reads of one hide the others')
+  for (int g0 = 0; g0 < Gt; g0 += 128) {
+    float v[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int gg = min(g0 + 64 * u + lane, Gt - 1);
+      v[u][0] = sc[wave * P + gg];
+      v[u][1] = two ? sc[(wave + kAttnWaves) * P + gg] : 0.0f;
+    }
+    const bool second = g0 + 64 < Gt;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (u == 1 && !second) break;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) v[u][k] = sfu_exp_np(v[u][k] - m, tab);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int gg = g0 + 64 * u + lane;
+      if (gg < Gt) {
+        sc[wave * P + gg] = gg * D + wave < T ? v[u][0] : 0.0f;
+        if (two) sc[(wave + kAttnWaves) * P + gg] = gg * D + wave + kAttnWaves < T ? v[u][1] : 0.0f;
       }
     }
   }
   lds_barrier();
   if (wave == 0) {
     float ssum = 0.0f;
-    if (lane < D) ssum = ordered_sum_t<false>(sc, T, D, P, lane);
+    if (lane < D) ssum = ordered_sum_long(sc, T, D, P, lane);
     if (lane == 0) s_r = (OPT && a.qsum) ? 1.0f : sfu_recip(ssum, tab);   // qsum: to_i8(F(F(e * 1) * 127))
   }
   lds_barrier();
@@ -769,9 +803,9 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
     constexpr int WP = (R / 4) * TS;             // words per pass
     const bool all = !SPLIT || (OPT && a.qsum);
     const int p0 = all ? 0 : sj, pst = all ? 1 : nsp;
-    const int nw = ((npass - p0 + pst - 1) / pst) * WP;
-    for (int q = tid; q < nw; q += kAttnThreads) {
+    for (int q = tid;; q += kAttnThreads) {
       const int ps = p0 + (q / WP) * pst, r = q % WP;
+      if (ps >= npass) break;
       const int t0 = ps * TS * R + r % TS + 4 * TS * (r / TS);
       float sv[4];
 #pragma unroll
@@ -792,7 +826,8 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
   int acc[16];
 #pragma unroll
   for (int b = 0; b < 16; ++b) acc[b] = 0;
-  for (int pass = sj; pass < npass; pass += nsp) {
+  int pass = sj;
+  for (; pass < npass; pass += nsp) {
     const int base = pass * TS * R;
     if (pass > sj) {
 #pragma unroll
@@ -818,7 +853,7 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
   }
   // row pos's term, p(pos) times the new V row (from LDS), in the threads whose slot holds row pos
   // (exact int32 either way)
-  if (ts == pos % TS && cok && (pos / (TS * R)) % nsp == sj) {
+  if (ts == pos % TS && cok && pass - nsp == npass - 1) {   // (row pos is in the last pass)
     const int ppos = to_i8((sc[osum_index(pos, D, P)] * rr) * 127.0f);
 #pragma unroll
     for (int w = 0; w < 4; ++w)
@@ -842,7 +877,8 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
   }
   if ((lane & 15) < NCHP && cok) {
 #pragma unroll
-    for (int b = 0; b < 16; ++b) part[wave * 4 + (lane >> 4)][16 * c + b] = acc[b];
+    for (int b = 0; b < 16; b += 4)
+      *(v4i_t*)&part[wave * 4 + (lane >> 4)][16 * c + b] = v4i_t{acc[b], acc[b + 1], acc[b + 2], acc[b + 3]};
   }
   __syncthreads();
   float* out = a.att + row * a.att_stride;
@@ -864,7 +900,8 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
     if (!pos_ok && tid == 0) flag_bad_pos(a.status);
     return;
   }
-  if constexpr (SPLIT == 1) {
+  const bool met = SPLIT == 1 && nsp > 1;          // the sums met with other splits'
+  if (met) {
     // this split's sums into the head's (exact int32 device atomics, every wave's complete before the
     // barrier); the last split to arrive finishes the output from them and clears them and the
     // counters for the next launch
@@ -885,7 +922,7 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
   if (!pos_ok && tid == 0) flag_bad_pos(a.status);   // (SPLIT 1 still clears its sums below)
   for (int j = tid; j < HD; j += kAttnThreads) {
     int ssum = 0;
-    if constexpr (SPLIT) {
+    if (met) {
       int* o = a.sp_acc + (long long)h * kMaxHd + j;
       ssum = __hip_atomic_load(o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(o, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -902,7 +939,7 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
       out[(long long)h * HD + j] = (float)ssum * a.a_v;
     }
   }
-  if (SPLIT && tid == 0) __hip_atomic_store(a.sp_sync + 2 * h + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (met && tid == 0) __hip_atomic_store(a.sp_sync + 2 * h + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---- prefill prep (ATTN_PREP): one wave per head vector of a row (the H query heads, then the Hk
@@ -2502,7 +2539,7 @@ __global__ __launch_bounds__(kGqaThreads) void k_attn_gqa(AttnArgs a) {
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 31, kh = lane >> 5;
   const int G = a.H / a.Hk, S = a.S, D = a.D, P = osum_stride(S, D), SH = D * P + 64;
   const int NSPL = G / GW;                       // workgroups per KV head
-  const int g = (int)blockIdx.x / NSPL, spl = (int)blockIdx.x - g * NSPL;
+  const int bx = xcd_col(blockIdx.x, gridDim.x), g = bx / NSPL, spl = bx - g * NSPL;
   const int GH = GW;                             // query heads of this workgroup
   const int h0 = g * G + spl * GW;               // its first query head
   const int SP = (S + 15) & ~15;                 // int8 p row stride
@@ -2731,7 +2768,7 @@ __global__ __launch_bounds__(kGqaThreads) void k_attn_gqa(AttnArgs a) {
   __syncthreads();
   if (wave < GH) {
     float ssum = 0.0f;
-    if (lane < D) ssum = ordered_sum_t<false>(dyn + wave * SH, T, D, P, lane);
+    if (lane < D) ssum = ordered_sum_long(dyn + wave * SH, T, D, P, lane);
     if (lane == 0) s_r[wave] = (OPT && a.qsum) ? 1.0f : sfu_recip(ssum, tab);   // qsum: to_i8(F(F(e * 1) * 127))
   }
   __syncthreads();
