@@ -202,9 +202,10 @@ int attn_launch(int mode, const AttnArgs& a, int rows, hipStream_t st) {
   // batched decode: per (row, KV head) its group of 2..4 query heads, over G / gw workgroups
   const int G = a.H / a.Hk;
   const bool opt = attn_opt(a);                 // the HF options: the kernels' OPT instantiations
-  // the group split over workgroups: two query heads each for four-head groups, else one
-  // (G / gw workgroups per KV head), each with its gw heads' score rows in LDS
-  const int gw = G == 4 ? 2 : 1;
+  // the group split over workgroups, each with its gw heads' score rows in LDS: one query head each while
+  // that gives every workgroup a CU of its own (C4, 8 rows: 902 us a step against 939), else two for four-head
+  // groups (16 rows: 1170 against 1261; 32 rows 1415 against 1694: K and V read half as often)
+  const int gw = G == 4 && (long long)rows * a.H > 256 ? 2 : 1;
   if (mode == ATTN_FUSED && rows > 1 && a.tab != nullptr && G >= 2 && G <= kGqaMaxG &&
       (a.hd == 64 || a.hd == 128) && attn_gqa_lds_bytes(a.S, a.D, gw) <= kGqaMaxLds) {
     const dim3 gs(a.Hk * (G / gw), rows);

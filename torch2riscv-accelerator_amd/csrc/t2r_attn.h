@@ -2533,7 +2533,7 @@ __global__ __launch_bounds__(kGqaThreads) void k_attn_gqa(AttnArgs a) {
   __shared__ float s_sq[GW], s_r[GW];
   __shared__ float red[kGqaWaves][GW];
   __shared__ int s_qs[kGqaWaves][GW];
-  __shared__ int part[kGqaWaves * 4][GW * HD];
+  __shared__ __align__(16) int part[kGqaWaves * 4][GW * HD];
 
   const int row = blockIdx.y, tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 31, kh = lane >> 5;
@@ -2725,7 +2725,7 @@ __global__ __launch_bounds__(kGqaThreads) void k_attn_gqa(AttnArgs a) {
         const bool ok = h < GH && t < T;
         const float sv = ((float)acc[r] * sqh[r]) * a.a_k;
         dyn[ok ? h * SH + osum_index(t, D, P) : (r < GH ? r : 0) * SH + D * P + lane] = sv;   // (spare slot)
-        mloc[r] = nanmax(mloc[r], ok ? sv : -__builtin_inff());
+        mloc[r] = smax(mloc[r], ok ? sv : -__builtin_inff());
       }
     }
   }
@@ -2733,13 +2733,13 @@ __global__ __launch_bounds__(kGqaThreads) void k_attn_gqa(AttnArgs a) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     float v = mloc[r];
-    v = nanmax(v, dpp_f<kDppXor1>(v));
-    v = nanmax(v, dpp_f<kDppXor2>(v));
-    v = nanmax(v, dpp_f<kDppHalfMirror>(v));
-    v = nanmax(v, dpp_f<kDppMirror>(v));
+    v = smax(v, dpp_f<kDppXor1>(v));
+    v = smax(v, dpp_f<kDppXor2>(v));
+    v = smax(v, dpp_f<kDppHalfMirror>(v));
+    v = smax(v, dpp_f<kDppMirror>(v));
     const float m0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
     const float m1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
-    if (lane == 0 && r < GH) red[wave][r] = nanmax(m0, m1);
+    if (lane == 0 && r < GH) red[wave][r] = smax(m0, m1);
   }
   __syncthreads();
 
@@ -2751,19 +2751,29 @@ __global__ __launch_bounds__(kGqaThreads) void k_attn_gqa(AttnArgs a) {
     const int h = r < GH ? r : 0;
     float m = red[0][h];
 #pragma unroll
-    for (int w = 1; w < kGqaWaves; ++w) m = nanmax(m, red[w][h]);
+    for (int w = 1; w < kGqaWaves; ++w) m = smax(m, red[w][h]);
     mh[r] = m;
   }
-  for (int t = tid; t < Tpad; t += kGqaThreads) {
-    const int k = osum_index(t, D, P);
-    float sv[GW], ev[GW];
+  for (int t0 = 0; t0 < Tpad; t0 += 2 * kGqaThreads) {   // (two keys a thread side by side)
+    float ev[2][GW];
 #pragma unroll
-    for (int h = 0; h < GW; ++h) sv[h] = dyn[(h < GH ? h : 0) * SH + k];
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
-    for (int h = 0; h < GW; ++h) ev[h] = sfu_exp_np(sv[h] - mh[h], tab);
+      for (int h = 0; h < GW; ++h) ev[u][h] = dyn[h * SH + osum_index(min(t0 + u * kGqaThreads + tid, Tpad - 1), D, P)];
+    const bool second = t0 + kGqaThreads < Tpad;
 #pragma unroll
-    for (int h = 0; h < GW; ++h)
-      if (h < GH) dyn[h * SH + k] = t < T ? ev[h] : 0.0f;
+    for (int u = 0; u < 2; ++u) {
+      if (u == 1 && !second) break;
+#pragma unroll
+      for (int h = 0; h < GW; ++h) ev[u][h] = sfu_exp_np(ev[u][h] - mh[h], tab);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int t = t0 + u * kGqaThreads + tid;
+      if (t < Tpad)
+#pragma unroll
+        for (int h = 0; h < GW; ++h) dyn[h * SH + osum_index(t, D, P)] = t < T ? ev[u][h] : 0.0f;
+    }
   }
   __syncthreads();
   if (wave < GH) {
@@ -2858,7 +2868,8 @@ __global__ __launch_bounds__(kGqaThreads) void k_attn_gqa(AttnArgs a) {
     for (int h = 0; h < GW; ++h)
       if (h < GH)
 #pragma unroll
-        for (int b = 0; b < 16; ++b) part[wave * 4 + (lane >> 4)][h * HD + 16 * c + b] = acc[h][b];
+        for (int b = 0; b < 16; b += 4)
+          *(v4i_t*)&part[wave * 4 + (lane >> 4)][h * HD + 16 * c + b] = v4i_t{acc[h][b], acc[h][b + 1], acc[h][b + 2], acc[h][b + 3]};
   }
   __syncthreads();
   if (!pos_ok) {

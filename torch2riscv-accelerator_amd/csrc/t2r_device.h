@@ -754,46 +754,47 @@ T2R_DEV float ordered_sum_t_all(const float* buf, int n, int D, int P, int l) {
   return lane_tree_sum(acc, D, l);
 }
 
-// ordered_sum_t (no squares) for the decode attention's long runs, whose other waves wait for it: sets of 32
-// values take turns, one requested while the other is added, and the last G % 32 are requested before the
-// first add, as pieces of 16, 8, 4, 2 and 1 (a 6100-position row's 381 values a lane took 2.8 us with 16
-// ahead and the last G % 16 read one by one). The values must not be -0 (EXPs are not: the chain starts
-// from +0). Reads up to 11 floats past the last lane's P.
+// ordered_sum_t (no squares) for the decode attention's long runs, whose other waves wait for it: three sets
+// of 16 values take turns, two requested ahead of the one being added, and the last G % 16 are requested
+// before the first add, as pieces of 8, 4, 2 and 1 (a 6100-position row's 381 values a lane: 1.8 us, against
+// 2.8 with one set ahead and the last ones read one by one; sets of 32 took the kernels past 128 registers,
+// one workgroup a CU). The values must not be -0 (EXPs are not: the chain starts from +0). Reads up to 4
+// floats past the last lane's P.
 T2R_DEV float ordered_sum_long(const float* buf, int n, int D, int P, int l) {
   const int G = n > 0 ? (n + D - 1) / D : 1;
   const float* row = buf + l * P;
-  const int nf = G >> 5, r = G & 31;
-  const float* t16 = row + 32 * nf;
-  const float* t8 = t16 + (r & 16);
+  const int nf = G >> 4, r = G & 15;
+  const float* t8 = row + 16 * nf;
   const float* t4 = t8 + (r & 8);
   const float* t2 = t4 + (r & 4);
-  v4f_t c[2][8], e16[4], e8[2];
+  v4f_t c0[4], c1[4], c2[4], e8[2];
   auto load = [&](v4f_t* d, int b) {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) d[q] = *(const v4f_t*)(row + 32 * b + 4 * q);
+    for (int q = 0; q < 4; ++q) d[q] = *(const v4f_t*)(row + 16 * b + 4 * q);
   };
   float acc = 0.0f;
   auto add = [&](const v4f_t* v, int nq) {
 #pragma unroll
     for (int q = 0; q < nq; ++q) acc = (((acc + v[q].x) + v[q].y) + v[q].z) + v[q].w;
   };
-  if (nf > 0) load(c[0], 0);
-  if (r & 16)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) e16[q] = *(const v4f_t*)(t16 + 4 * q);
+  if (nf > 0) load(c0, 0);
+  if (nf > 1) load(c1, 1);
 #pragma unroll
   for (int q = 0; q < 2; ++q) e8[q] = *(const v4f_t*)(t8 + 4 * q);
   const v4f_t e4 = *(const v4f_t*)t4;
   const float e2a = t2[0], e2b = t2[1], e1 = t2[r & 2];
-  for (int b = 0; b < nf; b += 2) {
-    if (b + 1 < nf) load(c[1], b + 1);
-    add(c[0], 8);
+  for (int b = 0; b < nf; b += 3) {
+    if (b + 2 < nf) load(c2, b + 2);
+    add(c0, 4);
     if (b + 1 < nf) {
-      if (b + 2 < nf) load(c[0], b + 2);
-      add(c[1], 8);
+      if (b + 3 < nf) load(c0, b + 3);
+      add(c1, 4);
+    }
+    if (b + 2 < nf) {
+      if (b + 4 < nf) load(c1, b + 4);
+      add(c2, 4);
     }
   }
-  if (r & 16) add(e16, 4);
   if (r & 8) add(e8, 2);
   if (r & 4) add(&e4, 1);
   if (r & 2) acc = (acc + e2a) + e2b;
