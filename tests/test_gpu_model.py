@@ -158,6 +158,27 @@ def test_moe_grouped_prefill_many_routes():
     rm.close()
 
 
+@pytest.mark.parametrize("rows,experts,k", [(9, 8, 4), (1100, 8, 4), (530, 64, 8)])
+def test_moe_route_groups(rows, experts, k):
+    """Route lists and groups of 32 at their ends: fewer routes than experts' groups, more than the list
+    kernel's ids in one step (4096), 64 experts with some unused: one call of the grouped path equals chunks of
+    7 rows, which take the per-row kernels."""
+    import t2r_amd.config as C
+    cfg = C.TINY_MOE.with_(name=f"tiny-moe-{rows}", seq_len=1104, n_experts=experts, top_k=k, prompt_len=rows)
+    qm, rm = resident(cfg, max_rows=rows)
+    toks = cfg.prompt()
+    print(f"{cfg.name}: {rows} rows, {experts} experts", flush=True)
+    a = rm.prefill(toks).cpu().numpy()
+    ka = kv_host(rm, rows)
+    rm.reset()
+    for i in range(0, rows, 7):
+        b = rm.prefill(toks[i:i + 7], start=i)
+    kb = kv_host(rm, rows)
+    assert sha(a) == sha(b.cpu().numpy())
+    assert np.array_equal(ka[0], kb[0]) and np.array_equal(ka[1], kb[1])
+    rm.close()
+
+
 def test_greedy_on_device_c1(gold):
     """The config-1 run as LlamaDevice.greedy_on_device does it (prefill, then argmax and pos += 1 on the
     device, no host round trip): the same 160 tokens as the reference's run."""

@@ -355,7 +355,6 @@ struct Model {
   uint32_t* sp_sync;
   // MoE over many rows, grouped by expert: route lists, the routes' int8 expert outputs and scales,
   // and their weighted down projections (MoE models only)
-  int32_t* moe_off = nullptr;
   int32_t* moe_list = nullptr;
   int8_t* moe_hq = nullptr;
   float* moe_sh = nullptr;
@@ -444,7 +443,6 @@ long long carve(Model* m, char* base, int M, char* state = nullptr, bool ext_sta
   m->pos_rows = c.take<int32_t>(M);
   if (d.n_experts > 0) {
     const long long routes = (long long)M * k;
-    m->moe_off = c.take<int32_t>(d.n_experts + 1);
     m->moe_list = c.take<int32_t>(routes);
     m->moe_hq = c.take<int8_t>(routes * d.hidden);
     m->moe_sh = c.take<float>(routes);
@@ -814,17 +812,19 @@ int run_layer(Model* m, int l, int rows, const int32_t* pos, int mode, hipStream
       {
         ProfScope p(m, T2R_PROF_ROUTE, st);
         route_rows();
-        launch(k_moe_lists, dim3(1), dim3(256), 0, st, (const int32_t*)m->ids, rows * k, E, m->moe_off, m->moe_list);
+        launch(k_moe_lists, dim3(1), dim3(kListThreads), 0, st, (const int32_t*)m->ids, rows * k, E, (v4i_t*)m->part, m->moe_list);
         if ((rc = launched())) return rc;
       }
       MoeGemmArgs g;
       std::memset(&g, 0, sizeof(g));
-      g.off = m->moe_off; g.list = m->moe_list; g.k = k; g.tab = sfu_table_ptr(); g.act = d.ffn_act;
-      g.ngrp = cdiv(rows, 32);                      // an expert takes at most one route of each row
+      // (the routes' groups lie in the linears' partial sums, which nothing holds here: fin_flush above;
+      // 16 (1 + E + rows k / 32) bytes of at least 16 rows dim)
+      g.groups = (const v4i_t*)m->part; g.list = m->moe_list; g.k = k; g.tab = sfu_table_ptr(); g.act = d.ffn_act;
+      const int max_groups = E + rows * k / 32;     // an expert's last group may hold fewer than 32 routes
       auto go = [&](auto mode, int K) {
         constexpr int MODE = decltype(mode)::value;
         const int nw = cdiv(K, kBgWin);
-        const dim3 grid((unsigned)((long long)E * g.ntile * g.ngrp));
+        const dim3 grid((unsigned)(8LL * cdiv(max_groups, 8) * g.ntile));
         if (nw >= 8) launch((k_moe_gemm<MODE, 8>), grid, dim3(512), 8 * kBgWaveLds, st, g);
         else if (nw >= 4) launch((k_moe_gemm<MODE, 4>), grid, dim3(256), 4 * kBgWaveLds, st, g);
         else if (nw >= 2) launch((k_moe_gemm<MODE, 2>), grid, dim3(128), 2 * kBgWaveLds, st, g);

@@ -264,19 +264,27 @@ __global__ __launch_bounds__(256) void k_kv_append(const float* k, const float* 
 // an equal value before a larger id; NaN scores after every number. Then the route weights
 // e = EXP(F(v - v0)), w = F(e * RECIP(red_sum(e))) (compiler/frontend/hf_generic.py:641-646).
 // Run by lanes [0, 64) of wave 0; sc in LDS.
-T2R_DEV bool route_before(float a, int ia, float b, int ib) {
-  const bool na = a != a, nb = b != b;
-  if (na || nb) return nb && (!na || ia < ib);
-  if (a != b) return a > b;
-  return ia < ib;
+// key: a larger key is placed first (NaN below every number, -0 equal to +0, then the smaller id)
+T2R_DEV unsigned long long route_key(float v, int id) {
+  uint32_t b = fb(v);
+  if ((b & 0x7FFFFFFFu) == 0) b = 0;
+  b = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+  b = v != v ? 0u : b;
+  return ((unsigned long long)b << 32) | (unsigned long long)(0xFFFFFFFFu - (uint32_t)id);
 }
 
 T2R_DEV void route_topk(const float* sc, int E, int k, int D, int lane, int32_t* ids, float* w, float* ev,
                         const float* tab = c_sfu) {
-  // lane e's rank: how many experts come before it under route_before (a total order: ids differ)
+  // lane e's rank: how many experts come before it, each lane's key read by every lane (a 12-instruction
+  // comparison with branches and one LDS read after another took most of the router's top-k)
   const float v = lane < E ? sc[lane] : 0.0f;
+  const unsigned long long key = lane < E ? route_key(v, lane) : 0ull;   // (0: below every expert's)
   int rank = 0;
-  for (int j = 0; j < E; ++j) rank += route_before(sc[j], j, v, lane) ? 1 : 0;
+  for (int j = 0; j < E; ++j) {
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(key >> 32), j);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)key, j);
+    rank += (((unsigned long long)hi << 32) | lo) > key ? 1 : 0;
+  }
   const bool sel = lane < E && rank < k;
   if (sel && rank == 0) ev[8] = v;                 // the top score v0
   __builtin_amdgcn_wave_barrier();
@@ -488,26 +496,52 @@ __global__ __launch_bounds__(kGemvThreads) void k_moe_up(MoeUpArgs m) {
 // 32 routes by an int8 MFMA tile (k_bgemv's main loop with the activation rows gathered through the
 // list). The int32 sums are exact, and every float step is the per-row kernels' own, in their order.
 
-// list[off[e] .. off[e + 1]) = the entries routed to expert e (in no particular order: each entry's
-// result is computed on its own). One workgroup; E <= 64.
-__global__ __launch_bounds__(256) void k_moe_lists(const int32_t* ids, int n, int E, int32_t* off, int32_t* list) {
+// list = the entries, expert by expert (within an expert in no particular order: each entry's result is
+// computed on its own), and groups: groups[0].x of them follow, each {expert, first list entry, routes <= 32},
+// in expert order. One workgroup; E <= 64. Bound by its round trips: four ids a thread requested together, a
+// wave's prefix sum (2664 routes: 3.6 us; 6.7 with 256 threads, an id at a time and a serial prefix).
+constexpr int kListThreads = 1024;
+__global__ __launch_bounds__(kListThreads) void k_moe_lists(const int32_t* ids, int n, int E, v4i_t* groups, int32_t* list) {
   __shared__ int cnt[64], fill[64];
+  constexpr int NP = 4;                            // ids a thread requests together
   const int tid = threadIdx.x;
   if (tid < 64) cnt[tid] = 0;
   __syncthreads();
-  for (int i = tid; i < n; i += 256) atomicAdd(&cnt[min(max(ids[i], 0), E - 1)], 1);
-  __syncthreads();
-  if (tid == 0) {
-    int o = 0;
-    for (int e = 0; e < E; ++e) {
-      off[e] = o;
-      fill[e] = o;
-      o += cnt[e];
-    }
-    off[E] = o;
+  for (int i0 = tid; i0 < n; i0 += NP * kListThreads) {
+    int id[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) id[p] = min(max(ids[min(i0 + p * kListThreads, n - 1)], 0), E - 1);
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+      if (i0 + p * kListThreads < n) atomicAdd(&cnt[id[p]], 1);
   }
   __syncthreads();
-  for (int i = tid; i < n; i += 256) list[atomicAdd(&fill[min(max(ids[i], 0), E - 1)], 1)] = i;
+  if (tid < 64) {                                  // the experts' first entries: a prefix sum over the wave
+    const int c = tid < E ? cnt[tid] : 0;
+    int o = c;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int u = __shfl_up(o, d);
+      o += tid >= d ? u : 0;
+    }
+    const int ng = (c + 31) >> 5;                  // the expert's groups of 32 routes, experts in order
+    int og = ng;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int u = __shfl_up(og, d);
+      og += tid >= d ? u : 0;
+    }
+    if (tid < E) fill[tid] = o - c;
+    for (int q = 0; q < ng; ++q) groups[1 + og - ng + q] = v4i_t{tid, o - c + 32 * q, min(32, c - 32 * q), 0};
+    if (tid == 63) groups[0] = v4i_t{og, 0, 0, 0};
+  }
+  __syncthreads();
+  for (int i0 = tid; i0 < n; i0 += NP * kListThreads) {
+    int id[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) id[p] = min(max(ids[min(i0 + p * kListThreads, n - 1)], 0), E - 1);
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+      if (i0 + p * kListThreads < n) list[atomicAdd(&fill[id[p]], 1)] = i0 + p * kListThreads;
+  }
 }
 
 // quant_act of every route's expert output u_j (one wave per entry; k_moe_down's prologue): hq [n, F]
@@ -535,15 +569,19 @@ __global__ __launch_bounds__(256) void k_moe_hq(const float* u, int n, int F, in
   if (lane == 0) s_h[ent] = sj;
 }
 
-// The grouped expert linear. Block b = (expert e, weight tile, route group g) takes the routes
-// list[off[e] + 32 g ..] (at most 32; a group past the expert's routes ends at once):
+// The grouped expert linear. A block takes one weight tile for one group of at most 32 routes of an expert
+// (list[beg ..], from k_moe_lists' groups). Each XCD takes an eighth of the groups, in expert order, so the
+// groups of an expert find its weights in that XCD's L2. Bound by each block's chain of dependent loads
+// (group, route, row; scales) around 32 KB of weights; C5, 333 rows: gate / up 28.1 -> 22.5 us, down 19.3 -> 14.9,
+// against a block for each (expert, possible group) with the scales loaded after the sums. Keeping a tile's
+// weights in LDS over all of its expert's groups measured 41 and 30 us (a third of the blocks, each in series):
 //   MOE_GU (gate / up): X = mxq[r] (K = dim), tiles of 16 gate + the same 16 up rows of expert e,
 //          u[r][j F + n] = gate(F(F(f32(s1) s_wg) s_x[r]), F(F(f32(s3) s_wu) s_x[r]))
 //   MOE_DN (down): X = hq[r k + j] (K = F), tiles of 32 rows of wd[e] (dim x F),
 //          t[r k + j][n] = F(w[r k + j] F(F(f32(s) s_wd) s_h[r k + j]))
 enum { MOE_GU = 0, MOE_DN = 1 };
 struct MoeGemmArgs {
-  const int32_t* off;
+  const v4i_t* groups;        // k_moe_lists: groups[0].x groups follow, each {expert, first list entry, routes}
   const int32_t* list;
   const int8_t* xq;           // GU: mxq [rows, dim] (row r = entry / k); DN: hq [rows k, F] (row = entry)
   const float* s_x;           // GU: msx [rows]; DN: s_h [rows k]
@@ -556,7 +594,7 @@ struct MoeGemmArgs {
   const float* tab;           // SFU tables (GU's gate)
   int act;
   int k, N, K;                // N: weight rows per expert (GU: F; DN: dim), K: their length
-  int ntile, ngrp;            // weight tiles per expert, route groups per expert
+  int ntile;                  // weight tiles per expert
 };
 template <int MODE, int KW>
 __global__ __launch_bounds__(64 * KW) void k_moe_gemm(MoeGemmArgs a) {
@@ -564,10 +602,12 @@ __global__ __launch_bounds__(64 * KW) void k_moe_gemm(MoeGemmArgs a) {
   __shared__ __align__(16) float tab_lds[MODE == MOE_GU ? kSfuWords : 4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lr = lane & 31, kh = lane >> 5;
-  const int per_e = a.ntile * a.ngrp;
-  const int e = blockIdx.x / per_e, tile = (blockIdx.x % per_e) / a.ngrp, grp = blockIdx.x % a.ngrp;
-  const int beg = a.off[e] + 32 * grp, cnt = min(32, a.off[e + 1] - beg);
-  if (cnt <= 0) return;                           // (block-uniform: before any barrier)
+  const int ngrp = a.groups[0].x, per = (ngrp + 7) >> 3;          // groups an XCD (blockIdx.x % 8) takes
+  const int slot = (int)(blockIdx.x >> 3) / a.ntile, tile = (int)(blockIdx.x >> 3) % a.ntile;
+  const int grp = (int)(blockIdx.x & 7) * per + slot;
+  if (slot >= per || grp >= ngrp) return;         // (block-uniform: before any barrier)
+  const v4i_t gr = a.groups[1 + grp];
+  const int e = gr.x, beg = gr.y, cnt = gr.z;
   constexpr int NT = MODE == MOE_GU ? 16 : 32;    // output columns per tile
   const int n0 = tile * NT, K = a.K, N = a.N;
   const int nwin = cdiv_i(K, kBgWin);
@@ -587,6 +627,24 @@ __global__ __launch_bounds__(64 * KW) void k_moe_gemm(MoeGemmArgs a) {
   // lane lr's activation row: route lr of the group (routes past cnt repeat the last one, unused)
   const int ent = a.list[beg + min(lr, cnt - 1)];
   const int8_t* xrow = a.xq + (long long)(MODE == MOE_GU ? ent / a.k : ent) * K + 16 * kh;
+  // the epilogue's route entries and scales, requested under the weight stream (output i of this thread:
+  // route m, column n)
+  constexpr int OPT = (32 * NT + 64 * KW - 1) / (64 * KW);
+  int em[OPT];
+  float sx[OPT], sw[OPT], sw3[OPT], wt[OPT];
+#pragma unroll
+  for (int i = 0; i < OPT; ++i) {
+    const int o = tid + i * 64 * KW;
+    em[i] = a.list[beg + min(o / NT, cnt - 1)];
+    const long long c = (long long)e * N + min(n0 + o % NT, N - 1);
+    sw[i] = a.s_w[c];
+    sw3[i] = MODE == MOE_GU ? a.s_w3[c] : 0.0f;
+  }
+#pragma unroll
+  for (int i = 0; i < OPT; ++i) {
+    sx[i] = a.s_x[MODE == MOE_GU ? em[i] / a.k : em[i]];
+    wt[i] = MODE == MOE_DN ? a.wts[em[i]] : 0.0f;
+  }
   v16i_t acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0;
@@ -614,7 +672,6 @@ __global__ __launch_bounds__(64 * KW) void k_moe_gemm(MoeGemmArgs a) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) red[((r >> 2) * 8 + kh * 4 + (r & 3)) * 33 + lr] = acc[r];
   __syncthreads();
-  constexpr int OPT = (32 * NT + 64 * KW - 1) / (64 * KW);
 #pragma unroll
   for (int i = 0; i < OPT; ++i) {
     const int o = tid + i * 64 * KW, m = o / NT, j = o % NT, n = n0 + j;
@@ -626,14 +683,10 @@ __global__ __launch_bounds__(64 * KW) void k_moe_gemm(MoeGemmArgs a) {
       s1 += rv[m * 33 + j];
       if (MODE == MOE_GU) s3 += rv[m * 33 + 16 + j];
     }
-    const int em = a.list[beg + m];
     if constexpr (MODE == MOE_GU) {
-      const int r = em / a.k, slot = em - r * a.k;
-      const float sx = a.s_x[r];
-      a.y[((long long)r * a.k + slot) * N + n] =
-          gate_mul(dequant(s1, a.s_w[(long long)e * N + n], sx), dequant(s3, a.s_w3[(long long)e * N + n], sx), a.act, tab_lds);
+      a.y[(long long)em[i] * N + n] = gate_mul(dequant(s1, sw[i], sx[i]), dequant(s3, sw3[i], sx[i]), a.act, tab_lds);
     } else {
-      a.y[(long long)em * N + n] = a.wts[em] * dequant(s1, a.s_w[(long long)e * N + n], a.s_x[em]);
+      a.y[(long long)em[i] * N + n] = wt[i] * dequant(s1, sw[i], sx[i]);
     }
   }
 }
