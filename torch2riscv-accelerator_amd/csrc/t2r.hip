@@ -176,15 +176,16 @@ inline bool pw_takes(const AttnArgs& a) { return a.tab != nullptr && a.kv_row_st
 inline bool ps_takes(const AttnArgs& a) { return a.tab != nullptr && a.kv_row_stride == 0 && (a.hd == 128 || a.hd == 64); }
 
 // batch-1 decode attention split over workgroups per head (k_attn_dec's SPLIT forms): the heads of a
-// model whose shape takes it (caches of more than one pass of the kernel: 512 rows at head dim 128, 1024
-// at 64; 4 splits a head in at most 256 workgroups), else 0
+// model whose shape takes it (head dim 128, caches over 512 rows, 4 splits a head in at most 256
+// workgroups), else 0. Not head dim 64: with an 8192-position cache C4's step at 6100 positions took 693 us
+// split against 751, but at 100 positions 511 against 500, and a 9-head model's 641 against 616 (one split
+// working, the others' workgroups ending at once).
 constexpr int kSplits = 4;
 inline int split_heads(const t2r_model_desc& d) {
-  const bool passes = (d.head_dim == 128 && d.seq_len > 512) || (d.head_dim == 64 && d.seq_len > 2048);
-  return passes && d.heads * kSplits <= 256 ? d.heads : 0;
+  return d.head_dim == 128 && d.seq_len > 512 && d.heads * kSplits <= 256 ? d.heads : 0;
 }
 inline bool attn_split(const AttnArgs& a, int rows) {
-  return a.nsplit > 1 && rows == 1 && (a.hd == 128 || a.hd == 64) && a.sp_s && a.sp_o && a.sp_acc && a.sp_sync;
+  return a.nsplit > 1 && rows == 1 && a.hd == 128 && a.sp_s && a.sp_o && a.sp_acc && a.sp_sync;
 }
 // ... and whether it leaves its int32 P.V sums per split for the next linear (SPLIT 2) instead of att
 inline bool attn_split_to_linear(const AttnArgs& a, int rows) { return attn_split(a, rows) && !attn_opt(a); }
@@ -235,13 +236,8 @@ int attn_launch(int mode, const AttnArgs& a, int rows, hipStream_t st) {
     if (attn_split(a, rows)) {
       // (without the HF options the next linear adds the splits' sums: attn_split_to_linear)
       const dim3 gs(a.H, a.nsplit);
-      if (a.hd == 64) {
-        if (opt) launch((k_attn_dec<4, true, 1>), gs, block, dl, st, a);
-        else launch((k_attn_dec<4, false, 2>), gs, block, dl, st, a);
-      } else {
-        if (opt) launch((k_attn_dec<8, true, 1>), gs, block, dl, st, a);
-        else launch((k_attn_dec<8, false, 2>), gs, block, dl, st, a);
-      }
+      if (opt) launch((k_attn_dec<8, true, 1>), gs, block, dl, st, a);
+      else launch((k_attn_dec<8, false, 2>), gs, block, dl, st, a);
     } else if (opt) {
       switch (a.hd / 16) {
         case 1: launch((k_attn_dec<1, true>), grid, block, dl, st, a); break;
@@ -910,9 +906,7 @@ bool split_fits(const t2r_model_desc& d, int heads) {
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return false;
-  const void* k8[] = {(const void*)k_attn_dec<8, false, 2>, (const void*)k_attn_dec<8, true, 1>};
-  const void* k4[] = {(const void*)k_attn_dec<4, false, 2>, (const void*)k_attn_dec<4, true, 1>};
-  const auto& ks = d.head_dim == 64 ? k4 : k8;
+  const void* ks[] = {(const void*)k_attn_dec<8, false, 2>, (const void*)k_attn_dec<8, true, 1>};
   for (const void* k : ks) {
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, kAttnThreads, attn_dec_lds_bytes(d.seq_len, d.D)) !=

@@ -112,7 +112,7 @@ T2R_DEV void wave_mem_done() {
 // it sets bit 1 of *status and returns, so every workgroup reaches its end whatever happens. What the
 // caller reads after it from other workgroups it reads by agent-scope atomic loads, which no cache of this
 // XCD answers, so the wait needs no agent-scope acquire: that would drop the L2's K / V lines as well (C3's
-// decode step at 2000 positions 802 -> 794 us without it, C4's at 6100 692 -> 685).
+// decode step at 2000 positions 802 -> 794 us without it).
 T2R_DEV void split_wait(uint32_t* p, uint32_t want, int32_t* status) {
   for (int it = 0; it < (1 << 20); ++it) {
     if ((int32_t)(__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - want) >= 0) {
@@ -457,10 +457,7 @@ T2R_DEV int slot_group_sum(int v) {
 
 // SPLIT (batch-1 decode of long caches): grid y splits a head's keys, workgroup j taking passes
 // j, j + n, ... (n = min(nsplit, passes); the others end at once). One CU streams a head's K and V
-// at most ~95 GB/s (522 KB at head dim 128 and T = 2048; half of it at head dim 64, whose rows are half a
-// 128-byte line), so more CUs per head shorten that part. At head dim 64 n is 1 up to two passes (2048
-// positions): their stream costs less than the exchange (C4's step at 1500 positions 580 us in one
-// workgroup a head, 611 in two), past them it does not (at 6100: 692 us against 780 in one).
+// at most ~95 GB/s (522 KB at head dim 128 and T = 2048), so more CUs per head shorten that part.
 // Each split publishes its scores with device-coherent stores and arrives once; after one bounded
 // wait every split reads all T scores and forms the max, the EXPs, the ordered sum and RECIP itself
 // (the same bits in each), then the probabilities and P.V of its own passes. The splits past the
@@ -469,9 +466,8 @@ T2R_DEV int slot_group_sum(int v) {
 // writes the output and clears the sums and its counter for the next launch. SPLIT 2 (no HF
 // options): each split stores its own int32 sums (splits past the passes store zeros) and the next
 // linear's prologue adds the four and scales them (F(f32(sum) a_v), the output's own formula).
-// C4's decode step at 6100 positions: 844 us with one workgroup a head, its query heads' workgroups on
-// different XCDs and the chain's values read 16 ahead; 692 us split, a KV head's workgroups on one XCD
-// (xcd_col: 780 without) and 32 ahead; at 2000 positions 601 -> 567 us, at 600 518 -> 511.
+// A KV head's query heads run on one XCD (xcd_col) and the ordered sum's values are read 32 ahead: C4's decode
+// step at 100 / 600 / 2000 / 6100 positions 502 / 518 / 601 / 844 us before both, 500 / 510 / 568 / 751 after.
 template <int NCH, bool OPT = false, int SPLIT = 0>   // 16-byte chunks per head row: hd = 16 NCH; OPT: the HF options
 __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
   constexpr int HD = 16 * NCH;
@@ -544,8 +540,7 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
   const bool pos_ok = pos_in >= 0 && pos_in < S;
   const int pos = pos_ok ? pos_in : 0;
   const int T = pos + 1;
-  // splits with passes; head dim 64: one up to two passes, whose second costs less than the exchange
-  const int nsp = SPLIT && !(HD == 64 && T <= 2 * TS * R) ? min(a.nsplit, (T + TS * R - 1) / (TS * R)) : 1;
+  const int nsp = SPLIT ? min(a.nsplit, (T + TS * R - 1) / (TS * R)) : 1;   // splits with passes
   // SPLIT: splits past the number of passes end here (all of a launch's workgroups agree on it; SPLIT 2:
   // with zero sums)
   if (SPLIT && sj >= nsp) {
