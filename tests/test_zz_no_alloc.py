@@ -95,6 +95,27 @@ def c3_small():
                       seed_w=911, seed_p=912, prompt_len=530, weight_std=None, gain_std=0.1, emb_scale=4.0)
 
 
+def test_short_workspace_refused():
+    """A workspace one byte below t2r_model_workspace_bytes is T2R_ENOMEM, also where the split decode
+    attention's part is what does not fit; the size it gives is taken."""
+    import t2r_amd.config as C
+    from t2r_amd import abi
+    from t2r_amd import weights as W
+    from t2r_amd.model import ResidentModel
+    lib = abi.load()
+    for cfg in (c3_small(), C.get("tiny-gqa")):
+        rm = ResidentModel(W.QuantModel(cfg), max_rows=4)
+        d = abi.ModelDesc.from_buffer_copy(bytes(rm.desc))
+        n = lib.t2r_model_workspace_bytes(ctypes.byref(d), 4)
+        h = ctypes.c_void_p()
+        d.workspace_bytes = n - 1
+        assert lib.t2r_model_create(ctypes.byref(d), ctypes.byref(h)) == abi.T2R_ENOMEM and not h.value
+        d.workspace_bytes = n
+        assert lib.t2r_model_create(ctypes.byref(d), ctypes.byref(h)) == abi.T2R_OK
+        lib.t2r_model_destroy(h)
+        rm.close()
+
+
 def test_two_static_models_interleaved():
     """Two static models of different max_rows alive at once (each handle keeps its carried state, the
     status word and the split attention's counters, in its own part of the array; the rest is shared

@@ -339,12 +339,11 @@ struct Model {
   int8_t* mxq;
   float* msx;
   int32_t* status;
-  // batch-1 decode attention split over workgroups per head (nsplit > 1; 0 when the shape or the workspace does
-  // not take it or the device cannot hold a launch's workgroups at once): published scores [H, S] and SPLIT 2's
+  // batch-1 decode attention split over workgroups per head (nsplit > 1; 0 when the shape does not take
+  // it or the device cannot hold a launch's workgroups at once): published scores [H, S] and SPLIT 2's
   // per-split P.V sums [4, H, kMaxHd] (both within one step); SPLIT 1's met sums [H, kMaxHd] and the
   // arrival counters [H, 2], carried from launch to launch (zeroed at creation)
   int nsplit = 0;
-  int hs = 0;                       // heads the workspace holds split state for (0: no split)
   float* sp_s;
   int32_t* sp_o;
   int32_t* sp_acc;
@@ -418,7 +417,7 @@ long long carve(Model* m, char* base, int M, char* state = nullptr, bool ext_sta
   const t2r_model_desc& d = m->d;
   Carve c{base, 0}, cs{state, 0};
   Carve& st = ext_state ? cs : c;
-  const int hs = m->hs;
+  const int hs = split_heads(d);
   m->status = st.take<int32_t>(1);
   m->sp_sync = st.take<uint32_t>(2LL * hs);
   m->sp_acc = st.take<int32_t>((long long)hs * kMaxHd);
@@ -437,6 +436,8 @@ long long carve(Model* m, char* base, int M, char* state = nullptr, bool ext_sta
   m->mxq = c.take<int8_t>((long long)M * d.dim);
   m->msx = c.take<float>(M);
   m->pos_rows = c.take<int32_t>(M);
+  m->sp_s = c.take<float>((long long)hs * d.seq_len);
+  m->sp_o = c.take<int32_t>((long long)kSplits * hs * kMaxHd);
   if (d.n_experts > 0) {
     const long long routes = (long long)M * k;
     m->moe_list = c.take<int32_t>(routes);
@@ -447,12 +448,7 @@ long long carve(Model* m, char* base, int M, char* state = nullptr, bool ext_sta
   // split-K partial sums of the prefill linears: 4 splits of up to 2048 rows of the widest
   // STORE / RESID output (C3's 2032-row prompt: 133 MB)
   m->part_rows = M < 2048 ? M : 2048;
-  // ... which a decode step does not use: the split attention's scores and sums are in the same bytes
-  const long long part = 4LL * m->part_rows * (m->qkv_dim > d.dim ? m->qkv_dim : d.dim);
-  const long long sc = ((long long)hs * d.seq_len + 63) / 64 * 64, split = sc + (long long)kSplits * hs * kMaxHd;
-  m->part = c.take<int32_t>(part > split ? part : split);
-  m->sp_s = (float*)m->part;
-  m->sp_o = m->part ? m->part + sc : nullptr;
+  m->part = c.take<int32_t>(4LL * m->part_rows * (m->qkv_dim > d.dim ? m->qkv_dim : d.dim));
   return c.off;
 }
 
@@ -466,7 +462,6 @@ void model_dims(Model* m) {
   if (m->q_dim > mi) mi = m->q_dim;
   if (d.hidden > mi) mi = d.hidden;
   m->max_in = mi;
-  m->hs = split_heads(d);
 }
 
 // the caller's descriptor as the current version: an ABI-1 descriptor ends before the HF options,
@@ -925,16 +920,10 @@ int model_init(Model* m, const t2r_model_desc& dv, char* state = nullptr, long l
   const t2r_model_desc* desc = &m->d;
   model_dims(m);
   long long sb = 0;
-  auto fits = [&]() {
-    return carve(m, nullptr, desc->max_rows, nullptr, state != nullptr, &sb) <= desc->workspace_bytes &&
-           sb <= (state ? state_cap : sb);
-  };
-  if (!fits()) {
-    m->hs = 0;                                       // a workspace that holds all but the split attention's part
-    if (!fits()) return T2R_ENOMEM;
-  }
+  if (carve(m, nullptr, desc->max_rows, nullptr, state != nullptr, &sb) > desc->workspace_bytes || sb > (state ? state_cap : sb))
+    return T2R_ENOMEM;
   carve(m, (char*)desc->workspace, desc->max_rows, state, state != nullptr);
-  const int hs = m->hs;
+  const int hs = split_heads(m->d);
   m->nsplit = hs > 0 && split_fits(m->d, hs) ? kSplits : 0;
   // the carried state starts clear: the status word, the split counters and SPLIT 1's sums
   if (hipMemset(m->status, 0, sizeof(int32_t)) != hipSuccess ||
