@@ -139,8 +139,9 @@ int t2r_attn_decode_opt(const float* q, const int8_t* kc, const int8_t* vc, cons
  * expandAttnChunkBlocked, compiler/plugins/sa/transforms/SahlExpandKernels.cpp:1702; QModel.prefill's
  * per-row attention, compiler/frontend/qhf.py:356-409). Each row's result is t2r_attn_decode_opt's for
  * that row, bit for bit; rows run 32 at a time per query head on int8 MFMA at hd 64 and 128, 16 at a time
- * where hd is another multiple of 16 (<= 128) and a row's scores fit in LDS, else row by row. Flags and per-channel scales as
- * t2r_attn_decode_opt. S = cache rows <= 8192. */
+ * where hd is another multiple of 16 (<= 128) and a row's scores fit in LDS, else row by row; 16 at a time or
+ * row by row also at hd 64 and 128 where that is faster (few rows past 2048 positions or with the options).
+ * Flags and per-channel scales as t2r_attn_decode_opt. S = cache rows <= 8192. */
 int t2r_attn_prefill(const float* q, const int8_t* kc, const int8_t* vc, const int32_t* pos, int M, int H, int Hk,
                      int hd, int S, float a_k, float a_v, int D, int flags, const float* ch_sk, const float* ch_av,
                      float* att, void* stream);

@@ -1,4 +1,5 @@
 import os
+import re
 import sys
 
 import pytest
@@ -25,3 +26,19 @@ def pytest_collection_modifyitems(config, items):
     for item in items:
         if "gpu" in item.keywords:
             item.add_marker(skip)
+
+
+@pytest.fixture
+def kernels():
+    """kernels(fn): the library's kernels that fn() launches, as torch's profiler names them
+    ("k_attn_ps<64, false>"); an empty set where the profiler reports none."""
+    def names(fn):
+        import torch
+        from torch.profiler import ProfilerActivity, profile
+        torch.cuda.synchronize()
+        with profile(activities=[ProfilerActivity.CUDA]) as p:
+            fn()
+            torch.cuda.synchronize()
+        found = (re.search(r"t2r::(k_\w+(?:<[^>]*>)?)\(", e.name) for e in p.events())
+        return {m.group(1) for m in found if m}
+    return names

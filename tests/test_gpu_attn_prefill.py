@@ -3,7 +3,8 @@ qhf.py:356-409) row by row against the CPU restatement (numerics.attention) and 
 on the same rows, bit for bit: consecutive prompt rows and scattered positions, head dims that take the
 multi-row MFMA kernel and ones that do not, GQA groups, D = 8 and 16, the HF options; and scores whose
 spread underflows EXP (x <= -104 gives +0) in the default instantiations of the prefill, decode and
-grouped decode kernels."""
+grouped decode kernels. Which kernel a call takes, on both sides of each line of the rule
+(test_attn_prefill_routes)."""
 import numpy as np
 import pytest
 
@@ -260,3 +261,63 @@ def test_attn_prefill_options_blocks(env, H_, Hk, hd, S, qsum, kch, vch):
         with np.errstate(invalid="ignore", over="ignore"):
             want = N.attention(q[i], kc[:p + 1], vc[:p + 1], H_, Hk, a_k, a_v, 16, qsum=qsum, ch_sk=ch_sk, ch_av=ch_av)
         assert np.array_equal(got[i].view(np.uint32), want.view(np.uint32)), f"row {i} pos {p}"
+
+
+# which kernel a call takes on both sides of each line of the rule, and its rows against the oracle: (heads, KV
+# heads, head dim, cache rows, rows, options, kernel)
+ROUTES = [
+    # past k_attn_pre's LDS: workgroups per (head, row) up to 512 / 448 of them, 256 with qsum, then streamed
+    (4, 2, 64, 2600, 8, "", "k_attn<"), (4, 2, 64, 2600, 128, "", "k_attn<"), (4, 2, 64, 2600, 129, "", "k_attn_ps<64, false>"),
+    (3, 1, 128, 2304, 149, "", "k_attn<"), (3, 1, 128, 2304, 150, "", "k_attn_ps<128, false>"),
+    (4, 2, 64, 2600, 64, "qsum", "k_attn<"), (4, 2, 64, 2600, 65, "qsum", "k_attn_ps<64, true>"),
+    (3, 1, 128, 2600, 85, "qsum+k", "k_attn<"), (3, 1, 128, 2600, 86, "qsum+k", "k_attn_ps<128, true>"),
+    (4, 2, 64, 8192, 130, "v", "k_attn_ps<64, true>"), (3, 1, 128, 8192, 161, "k+v", "k_attn_ps<128, true>"),
+    # within it: 16-row blocks
+    (4, 2, 64, 2080, 64, "", "k_attn_pre<64, false>"), (4, 2, 64, 2080, 65, "", "k_attn_ps<64, false>"),
+    (3, 1, 128, 2080, 33, "", "k_attn_pre<128, false>"),
+    (4, 2, 64, 64, 15, "v", "k_attn_pre<64, true>"), (4, 2, 64, 64, 16, "v", "k_attn_ps<64, true>"),
+    (4, 2, 64, 65, 15, "k", "k_attn_ps<64, true>"), (4, 2, 64, 64, 15, "qsum", "k_attn_ps<64, true>"),
+    (4, 2, 64, 512, 64, "k+v", "k_attn_ps<64, true>"), (4, 2, 64, 513, 64, "k+v", "k_attn_pre<64, true>"),
+    (4, 2, 64, 513, 65, "v", "k_attn_ps<64, true>"),
+    (4, 2, 128, 64, 15, "qsum", "k_attn_pre<128, true>"), (4, 2, 128, 64, 16, "qsum", "k_attn_ps<128, true>"),
+    (4, 2, 128, 65, 15, "qsum+k", "k_attn_ps<128, true>"),
+    (16, 8, 128, 300, 256, "v", "k_attn_pre<128, true>"), (16, 8, 128, 300, 257, "v", "k_attn_ps<128, true>"),
+    # other head dims with the options
+    (4, 2, 96, 700, 35, "k+v", "k_attn_pre<128, true>"), (4, 2, 80, 300, 17, "qsum", "k_attn_pre<128, true>"),
+    (2, 1, 112, 129, 16, "qsum+k", "k_attn_pre<128, true>"),
+    # scores kept in registers, without the options
+    (4, 2, 64, 512, 5, "", "k_attn_pw<64, 2, false>"), (4, 2, 64, 513, 5, "", "k_attn_pw<64, 8, false>"),
+    (3, 1, 128, 2048, 5, "", "k_attn_pw<128, 8, false>"),
+]
+
+
+# (the scale's sign and range matter to the streamed kernel's maxima)
+@pytest.mark.parametrize("H_,Hk,hd,S,M,opt,kernel,ak", [
+    (*r, ak) for r in ROUTES for ak in (0.02, -0.02, 0.0, np.inf)
+    if ak == 0.02 or (r[6].startswith("k_attn_ps") and "k" not in r[5])])
+def test_attn_prefill_routes(env, kernels, H_, Hk, hd, S, M, opt, kernel, ak):
+    """Rows at the edges of 32-key tiles and 256-key chunks and at the cache's end, the last two with a NaN and
+    an infinite q; the scores' scale positive, negative, zero and infinite."""
+    torch, N, ops, T, H = env
+    rng = np.random.default_rng(S + 7 * M + hd)
+    kc, vc = caches(rng, S, Hk * hd)
+    D = 8 if M % 2 else 16
+    pos = np.arange(S - M, S, dtype=np.int32)
+    if M >= 8:
+        pos[:4] = np.minimum([0, 31, 32, 255], S - 1)
+    q = (rng.standard_normal((M, H_ * hd)) * 2).astype(F)
+    q[-2, 1], q[-1, 3] = np.nan, np.inf
+    ch_sk = np.exp(rng.uniform(-4, 1, Hk * hd)).astype(F) * F(0.01) if "k" in opt else None
+    ch_av = np.exp(rng.uniform(-3, 2, Hk * hd)).astype(F) * F(1e-3) if "v" in opt else None
+    a_k, a_v = F((1.0 if ch_sk is not None else ak) / np.sqrt(hd)), F(0.03 / 127)
+    t = lambda a: None if a is None else T(a)
+    args = (T(q), T(kc), T(vc), T(pos), H_, Hk, a_k, a_v, D, "qsum" in opt, t(ch_sk), t(ch_av))
+    print(f"H {H_} hd {hd} S {S} D {D} {opt} a_k {a_k}: {M} rows", flush=True)
+    got = H(ops.attention_prefill(*args))
+    for i in sorted({0, 1, 2, 3, M // 2, M - 3, M - 2, M - 1}):
+        p = int(pos[i])
+        with np.errstate(invalid="ignore", over="ignore"):
+            want = N.attention(q[i], kc[:p + 1], vc[:p + 1], H_, Hk, a_k, a_v, D, qsum="qsum" in opt, ch_sk=ch_sk, ch_av=ch_av)
+        assert np.array_equal(got[i].view(np.uint32), want.view(np.uint32)), f"row {i} pos {p}"
+    ran = kernels(lambda: ops.attention_prefill(*args))
+    assert not ran or any(k.startswith(kernel) for k in ran), ran

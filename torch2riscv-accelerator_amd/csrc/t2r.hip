@@ -164,8 +164,8 @@ bool pre_ok(const AttnArgs& a) {
   return a.hd % 16 == 0 && a.hd <= 128 && attn_pre_lds_bytes(pre_cap(a), (a.hd + 31) & ~31) <= kPreMaxLds;
 }
 // ... and its 32-row form (k_attn_pw): head dims 128 and 64 without the HF options, rows attending to at
-// most the 2048 positions whose scores a block keeps in registers. Past them, and with the options, the
-// streamed form (ps_takes) is the faster one of what is left: see the kernels for both sides.
+// most the 2048 positions whose scores a block keeps in registers. Past them, and with the options: the
+// streamed form (k_attn_ps), where ps_takes has it as the faster one.
 bool pw_ok(const AttnArgs& a) {
   if (attn_opt(a) || !(a.D == 8 || a.D == 16)) return false;
   return (a.hd == 128 || a.hd == 64) && pre_cap(a) <= ap_keys<8>();
@@ -173,7 +173,27 @@ bool pw_ok(const AttnArgs& a) {
 // the multi-row ATTN_ONLY launch runs k_attn_pw (only then may q come as int8 rows: AttnArgs::q8)
 inline bool pw_takes(const AttnArgs& a) { return a.tab != nullptr && a.kv_row_stride == 0 && pw_ok(a); }
 
-inline bool ps_takes(const AttnArgs& a) { return a.tab != nullptr && a.kv_row_stride == 0 && (a.hd == 128 || a.hd == 64); }
+// ... and what pw_takes leaves runs k_attn_ps at head dims 64 / 128, but not for few rows: a block of 32 rows
+// walks its head's keys two or three times however few of the rows exist, on H cdiv(rows, 32) CUs.
+//  - Past k_attn_pre's LDS the other side is k_attn's workgroup per (head, row), the faster one while its
+//    workgroups are on the chip at once. C4 (32 heads of 64), 8 / 16 / 24 rows at 7000 positions: 40 / 70 / 103
+//    us, against 85 streamed; C3 (16 heads of 128), 8 / 24 / 32 rows: 56 / 110 / 133 against 120. With qsum the
+//    streamed form has one EXP a key and no chains: C4, 8 / 16 rows 40 / 69 against 47, C3 56 / 64 against 75.
+//  - Within it the other side is k_attn_pre's blocks of 16 rows. Without qsum at head dim 128 they win while each
+//    has a CU (C3, V per channel, 2048 positions: 256 rows 34.5 us against 45.0, 257 rows 59 against 45); at head
+//    dim 64 past 512 positions only while there are fewer rows and heads than CUs (9 heads, 8 / 28 rows: 27.1 /
+//    28.3 against 28.9 / 29.2; 32 heads, 8 / 15 rows: 28.9 / 30.2 against 28.8 / 29.0). Below 16 rows at up to 64
+//    positions the streamed form's longer prologue shows as well (C3, 4 rows: 7.3 us, 8.3 streamed with qsum,
+//    10.3 without), but for qsum at head dim 64 (7.5 against 6.5 streamed).
+inline bool ps_takes(const AttnArgs& a, int rows) {
+  if (a.tab == nullptr || a.kv_row_stride != 0 || (a.hd != 128 && a.hd != 64)) return false;
+  if (!pre_ok(a)) return (long long)rows * a.H > (a.qsum ? 256 : a.hd == 64 ? 512 : 448);
+  if (a.qsum && a.hd == 64) return true;
+  const int cap = pre_cap(a);
+  if (rows < kPreRows && cap <= 64) return false;
+  if (a.qsum) return true;
+  return a.hd == 128 ? (long long)a.H * cdiv(rows, kPreRows) > 256 : cap <= 512 || (long long)a.H * rows > 256;
+}
 
 // batch-1 decode attention split over workgroups per head (k_attn_dec's SPLIT forms): the heads of a
 // model whose shape takes it (head dim 128, caches over 512 rows, 4 splits a head in at most 256
@@ -281,7 +301,7 @@ int attn_launch(int mode, const AttnArgs& a, int rows, hipStream_t st) {
     } else {
       launch((k_attn_pw<64, 8, false>), grid_pw, dim3(kApThreads), ap_lds<64, 8>(), st, a, rows);
     }
-  } else if (ps_takes(a)) {
+  } else if (ps_takes(a, rows)) {
     const dim3 grid_ps(a.H, cdiv(rows, kApRows));
     if (a.hd == 128) {
       if (opt) launch((k_attn_ps<128, true>), grid_ps, dim3(kApThreads), as_lds<128>(), st, a, rows);
