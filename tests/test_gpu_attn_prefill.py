@@ -285,6 +285,9 @@ ROUTES = [
     # other head dims with the options
     (4, 2, 96, 700, 35, "k+v", "k_attn_pre<128, true>"), (4, 2, 80, 300, 17, "qsum", "k_attn_pre<128, true>"),
     (2, 1, 112, 129, 16, "qsum+k", "k_attn_pre<128, true>"),
+    # caches whose score rows take less LDS than the kernel's 16 x 128 P.V sums
+    (4, 2, 96, 40, 20, "", "k_attn_pre<128, false>"), (2, 1, 80, 33, 16, "", "k_attn_pre<128, false>"),
+    (4, 2, 96, 48, 33, "k+v", "k_attn_pre<128, true>"), (4, 2, 96, 49, 16, "qsum", "k_attn_pre<128, true>"),
     # scores kept in registers, without the options
     (4, 2, 64, 512, 5, "", "k_attn_pw<64, 2, false>"), (4, 2, 64, 513, 5, "", "k_attn_pw<64, 8, false>"),
     (3, 1, 128, 2048, 5, "", "k_attn_pw<128, 8, false>"),

@@ -160,8 +160,9 @@ int pre_cap(const AttnArgs& a) { return a.t_cap > 0 && a.t_cap < a.S ? a.t_cap :
 
 // the multi-row prefill attention: head dims 16..128 (multiples of 16), cache rows whose
 // score rows fit the LDS the kernels are set up for (kPreMaxLds)
+inline int pre_hdp(int hd) { return hd <= 32 ? 32 : hd <= 64 ? 64 : 128; }   // k_attn_pre's instantiation
 bool pre_ok(const AttnArgs& a) {
-  return a.hd % 16 == 0 && a.hd <= 128 && attn_pre_lds_bytes(pre_cap(a), (a.hd + 31) & ~31) <= kPreMaxLds;
+  return a.hd % 16 == 0 && a.hd <= 128 && attn_pre_lds_bytes(pre_cap(a), pre_hdp(a.hd)) <= kPreMaxLds;
 }
 // ... and its 32-row form (k_attn_pw): head dims 128 and 64 without the HF options, rows attending to at
 // most the 2048 positions whose scores a block keeps in registers. Past them, and with the options: the
@@ -311,7 +312,7 @@ int attn_launch(int mode, const AttnArgs& a, int rows, hipStream_t st) {
       else launch((k_attn_ps<64, false>), grid_ps, dim3(kApThreads), as_lds<64>(), st, a, rows);
     }
   } else if (a.tab != nullptr && a.kv_row_stride == 0 && pre_ok(a)) {
-    const int hdp = (a.hd + 31) & ~31;
+    const int hdp = pre_hdp(a.hd);
     dim3 pg(a.H, cdiv(rows, kPreRows));
     const size_t pl = attn_pre_lds_bytes(pre_cap(a), hdp);
     if (opt) {

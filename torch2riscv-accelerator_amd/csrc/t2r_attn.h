@@ -1667,7 +1667,7 @@ __global__ __launch_bounds__(pre_threads(HDP)) void k_attn_pre(AttnArgs a, int M
   }
 }
 
-// dynamic LDS bytes of k_attn_pre: 16 rows of scores / exps (also the P.V sums afterwards)
+// dynamic LDS bytes of k_attn_pre<HDP>: 16 rows of scores / exps (also the P.V sums [16][HDP] afterwards)
 inline size_t attn_pre_lds_bytes(int S, int HDP) {
   const size_t e = (size_t)kPreRows * pre_est(S) * 4, p = (size_t)kPreRows * HDP * 4;
   return e > p ? e : p;
