@@ -324,3 +324,35 @@ def test_attn_prefill_routes(env, kernels, H_, Hk, hd, S, M, opt, kernel, ak):
         assert np.array_equal(got[i].view(np.uint32), want.view(np.uint32)), f"row {i} pos {p}"
     ran = kernels(lambda: ops.attention_prefill(*args))
     assert not ran or any(k.startswith(kernel) for k in ran), ran
+
+
+@pytest.mark.parametrize("H_,Hk,hd,S,opt,kernel", [(4, 2, 64, 2600, "", "k_attn<"), (4, 2, 64, 600, "", "k_attn_pre<64, false>"),
+                                                   (4, 2, 64, 300, "qsum", "k_attn_pre<64, true>"),
+                                                   (3, 1, 128, 700, "", "k_attn_pre<128, false>"),
+                                                   (3, 1, 128, 300, "qsum", "k_attn_pre<128, true>")])
+@pytest.mark.parametrize("off", [(4, 4), (8, 0), (0, 4)])
+def test_attn_prefill_unaligned_caches(env, kernels, H_, Hk, hd, S, opt, kernel, off):
+    """Caches that start off a 16-byte boundary: the kernels that fetch tiles by 16-byte DMA do not take them.
+    131 rows: as many as the streamed kernel would take."""
+    torch, N, ops, T, H = env
+    rng = np.random.default_rng(S + hd)
+    M = 131
+    kc, vc = caches(rng, S, Hk * hd)
+
+    def at(a, o):                                  # the rows, o bytes into an allocation
+        flat = torch.zeros(a.size + 16, dtype=torch.int8, device="cuda:0")
+        t = flat[o:o + a.size].view(a.shape)
+        t.copy_(T(a))
+        return t
+    pos = np.arange(S - M, S, dtype=np.int32)
+    q = (rng.standard_normal((M, H_ * hd)) * 2).astype(F)
+    a_k, a_v = F(0.02 / np.sqrt(hd)), F(0.03 / 127)
+    args = (T(q), at(kc, off[0]), at(vc, off[1]), T(pos), H_, Hk, a_k, a_v, 16, "qsum" in opt)
+    print(f"hd {hd} S {S} {opt} caches at +{off}", flush=True)
+    got = H(ops.attention_prefill(*args))
+    for i in (0, 1, 64, M - 1):
+        p = int(pos[i])
+        want = N.attention(q[i], kc[:p + 1], vc[:p + 1], H_, Hk, a_k, a_v, 16, qsum="qsum" in opt)
+        assert np.array_equal(got[i].view(np.uint32), want.view(np.uint32)), f"row {i} pos {p}"
+    ran = kernels(lambda: ops.attention_prefill(*args))
+    assert not ran or any(k.startswith(kernel) for k in ran), ran

@@ -171,8 +171,13 @@ bool pw_ok(const AttnArgs& a) {
   if (attn_opt(a) || !(a.D == 8 || a.D == 16)) return false;
   return (a.hd == 128 || a.hd == 64) && pre_cap(a) <= ap_keys<8>();
 }
+// k_attn_pw and k_attn_ps fetch K and V by 16-byte DMA to LDS: one cache, its rows on 16-byte boundaries
+// (the other kernels' plain loads do not need them there)
+inline bool dma_ok(const AttnArgs& a) {
+  return a.tab != nullptr && a.kv_row_stride == 0 && (((uintptr_t)a.kc | (uintptr_t)a.vc) & 15) == 0;
+}
 // the multi-row ATTN_ONLY launch runs k_attn_pw (only then may q come as int8 rows: AttnArgs::q8)
-inline bool pw_takes(const AttnArgs& a) { return a.tab != nullptr && a.kv_row_stride == 0 && pw_ok(a); }
+inline bool pw_takes(const AttnArgs& a) { return dma_ok(a) && pw_ok(a); }
 
 // ... and what pw_takes leaves runs k_attn_ps at head dims 64 / 128, but not for few rows: a block of 32 rows
 // walks its head's keys two or three times however few of the rows exist, on H cdiv(rows, 32) CUs.
@@ -187,7 +192,7 @@ inline bool pw_takes(const AttnArgs& a) { return a.tab != nullptr && a.kv_row_st
 //    positions the streamed form's longer prologue shows as well (C3, 4 rows: 7.3 us, 8.3 streamed with qsum,
 //    10.3 without), but for qsum at head dim 64 (7.5 against 6.5 streamed).
 inline bool ps_takes(const AttnArgs& a, int rows) {
-  if (a.tab == nullptr || a.kv_row_stride != 0 || (a.hd != 128 && a.hd != 64)) return false;
+  if (!dma_ok(a) || (a.hd != 128 && a.hd != 64)) return false;
   if (!pre_ok(a)) return (long long)rows * a.H > (a.qsum ? 256 : a.hd == 64 ? 512 : 448);
   if (a.qsum && a.hd == 64) return true;
   const int cap = pre_cap(a);
