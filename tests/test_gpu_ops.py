@@ -360,6 +360,19 @@ def test_argmax_edges(env, n):
     assert list(got) == [int(np.argmax(r)) for r in x]
 
 
+def test_argmax_longest_row(env):
+    """A row of 2^31 - 1 values, the most the call takes: the last pass over it reaches past an int's range."""
+    torch, N, ops, T, H = env
+    n = 2**31 - 1
+    x = torch.zeros(n, dtype=torch.float32, device="cuda:0")
+    for at in (n - 1, n - 5, n - 32770, 3):           # (later ones come first in the row)
+        x[at] = 2.0
+        print(f"n {n}: largest value at {at}", flush=True)
+        assert int(ops.argmax(x.view(1, n))[0]) == at
+    del x
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("rows,n", [(3, 16), (2, 1024), (2, 1040), (3, 2048), (1, 4112), (2, 8192)])
 @pytest.mark.parametrize("off", [0, 1])
 def test_row_ops_alignment(env, rows, n, off):

@@ -799,23 +799,24 @@ __global__ __launch_bounds__(256) void k_moe_down(MoeDownArgs m) {
 constexpr int kArgmaxThreads = 1024;
 __global__ __launch_bounds__(kArgmaxThreads) void k_argmax(const float* x, int n, int32_t* idx) {
   typedef float v4u_t __attribute__((ext_vector_type(4), aligned(4)));   // (a row may start at any float)
-  constexpr int NP = 8, NW = kArgmaxThreads / 64, SPAN = 4 * kArgmaxThreads;
+  constexpr uint32_t NP = 8, NW = kArgmaxThreads / 64, SPAN = 4 * kArgmaxThreads;
   __shared__ float red[NW];
   __shared__ int ired[NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const float* xr = x + (long long)blockIdx.x * n;
   float best = -__builtin_inff();
-  int pass = 0;                                    // the first value of the pass that best came from
-  // loads past the row are clamped into it: they repeat values under their own index
-  auto at = [&](int i0, int p) { return min(i0 + SPAN * p + 4 * tid, n - 4); };
+  uint32_t pass = 0;                               // the first value of the pass that best came from
+  // loads past the row are clamped into it: they repeat values under their own index (unsigned: a pass of a
+  // row of nearly 2^31 values reaches past it)
+  auto at = [&](uint32_t i0, uint32_t p) { return (int)min(i0 + SPAN * p + 4u * tid, (uint32_t)n - 4); };
   if (n >= 4) {
-    for (int i0 = 0; i0 < n; i0 += NP * SPAN) {
+    for (uint32_t i0 = 0; i0 < (uint32_t)n; i0 += NP * SPAN) {
       v4u_t v[NP];
 #pragma unroll
-      for (int p = 0; p < NP; ++p) v[p] = *(const v4u_t*)(xr + at(i0, p));
+      for (uint32_t p = 0; p < NP; ++p) v[p] = *(const v4u_t*)(xr + at(i0, p));
       float m = smax(smax(v[0].x, v[0].y), smax(v[0].z, v[0].w));
 #pragma unroll
-      for (int p = 1; p < NP; ++p) m = smax(smax(m, smax(v[p].x, v[p].y)), smax(v[p].z, v[p].w));
+      for (uint32_t p = 1; p < NP; ++p) m = smax(smax(m, smax(v[p].x, v[p].y)), smax(v[p].z, v[p].w));
       if (m > best || (m != m && best == best)) {
         best = m;
         pass = i0;
@@ -835,7 +836,7 @@ __global__ __launch_bounds__(kArgmaxThreads) void k_argmax(const float* x, int n
       if (v == mx || (v != v && mx != mx)) first = min(first, i);
     };
     if (n >= 4) {
-      for (int p = 0; p < NP; ++p)
+      for (uint32_t p = 0; p < NP; ++p)
         for (int e = 0; e < 4; ++e) look(at(pass, p) + e);
     } else if (tid < n) {
       look(tid);
@@ -845,7 +846,7 @@ __global__ __launch_bounds__(kArgmaxThreads) void k_argmax(const float* x, int n
   if (lane == 0) ired[wave] = first;
   __syncthreads();
   if (tid == 0) {
-    for (int w = 1; w < NW; ++w) first = min(first, ired[w]);
+    for (uint32_t w = 1; w < NW; ++w) first = min(first, ired[w]);
     idx[blockIdx.x] = first;
   }
 }
