@@ -1,7 +1,7 @@
 """Long context: caches of 8192 positions (the datapath's kMaxS), past the 2048 of the measured
-configs. The decode kernels then take several passes over the keys, the prefill attention falls back
-to the per-(head, row) kernel when a chunk's score rows do not fit in LDS, and the batched step to
-per-head attention. Each is checked against the CPU restatement or the others, bit for bit."""
+configs. The decode kernels then take several passes over the keys (at head dim 128 split over workgroups,
+each with several passes), and prompts past 2048 positions the streamed prefill attention. Each is checked
+against the CPU restatement or the others, bit for bit."""
 import numpy as np
 import pytest
 
@@ -119,4 +119,39 @@ def test_c4_8k_paths_agree():
         want = rm.decode(nxt[b], lens[b]).cpu().numpy()
         assert np.array_equal(out[b].view(np.uint32), want.view(np.uint32)), f"batched row {b} at {lens[b]}"
         assert torch.equal(kc[b, :, lens[b]], rm.kc[:, lens[b]])
+    rm.close()
+
+
+@pytest.mark.parametrize("hf", [False, True])
+@pytest.mark.parametrize("D", [16, 8])
+def test_split_decode_8k(kernels, hf, D):
+    """Head dim 128, batch 1: each head's keys over four workgroups, at positions around 2048 (from where the
+    published scores are gathered eight at a time) and around whole numbers of 512-key passes a workgroup, over
+    random caches; without the options (the next linear adds the splits' sums) and with them (the splits meet)."""
+    import torch
+    import t2r_amd.config as C
+    from oracle import OracleModel
+    from t2r_amd import weights as W
+    from t2r_amd.model import ResidentModel
+    cfg = C.ModelConfig("small-8k-128", dim=256, hidden=256, layers=2, heads=4, kv_heads=2, head_dim=128, vocab=96, seq_len=8192,
+                        theta=1e6, qk_norm=True, D=D, weight_std=None, gain_std=0.1, emb_scale=4.0, seed_w=71, seed_p=72,
+                        prompt_len=32).validate()
+    cfg = C.hf_options(cfg) if hf else cfg
+    qm = W.QuantModel(cfg, kv_scales=W.calibrate_kv(cfg, tokens=cfg.prompt()))
+    om, rm = OracleModel(qm), ResidentModel(qm, max_rows=1)
+    rng = np.random.default_rng(73)
+    for t, o in ((rm.kc, om.kc), (rm.vc, om.vc)):
+        o[:] = np.clip(np.rint(rng.standard_normal(o.shape) * 28), -127, 127)
+        t.copy_(torch.from_numpy(o.astype(np.int8)))
+    for p in (0, 511, 512, 2047, 2048, 2049, 2560, 4095, 4096, 4097, 6143, 6144, 8191):
+        t = int(rng.integers(0, cfg.vocab))
+        print(f"{cfg.name} D {D}: decode at {p}", flush=True)
+        want = om.forward(t, p)
+        got = rm.decode(t, p).cpu().numpy()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), f"decode at {p}"
+        assert np.array_equal(rm.kc[:, p].cpu().numpy(), om.kc[:, p]) and np.array_equal(rm.vc[:, p].cpu().numpy(), om.vc[:, p])
+        rm.check_status(f"pos {p}")
+    assert np.array_equal(rm.kc.cpu().numpy(), om.kc) and np.array_equal(rm.vc.cpu().numpy(), om.vc)
+    ran = kernels(lambda: rm.decode(t, p))
+    assert not ran or ("k_attn_dec<8, true, 1>" if hf else "k_attn_dec<8, false, 2>") in ran, ran
     rm.close()
