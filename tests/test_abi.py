@@ -160,3 +160,33 @@ def test_hf_option_validation_before_launch():
     v1.attn_qsum = 7
     assert lib.t2r_model_workspace_bytes(ctypes.byref(v1), 4) == lib.t2r_model_workspace_bytes(
         ctypes.byref(_desc(cfg, 4)), 4)
+
+
+def _code_object_functions(so):
+    """{name: (address, size)} of the functions of the gfx950 code object inside the built library."""
+    import struct
+    blob = open(so, "rb").read()
+    out, at = {}, blob.find(b"\x7fELF", 1)
+    while at >= 0:
+        if struct.unpack_from("<H", blob, at + 18)[0] == 224:                # EM_AMDGPU
+            shoff, = struct.unpack_from("<Q", blob, at + 40)
+            size, num = struct.unpack_from("<HH", blob, at + 58)
+            sec = [struct.unpack_from("<IIQQQQIIQQ", blob, at + shoff + size * i) for i in range(num)]
+            for s in sec:
+                if s[1] != 11:                                              # SHT_DYNSYM
+                    continue
+                names = at + sec[s[6]][4]
+                for o in range(at + s[4], at + s[4] + s[5], 24):
+                    name, info, _, _, value, n = struct.unpack_from("<IBBHQQ", blob, o)
+                    if info & 15 == 2:                                      # STT_FUNC
+                        out[blob[names + name:blob.index(0, names + name)].decode()] = (value, n)
+        at = blob.find(b"\x7fELF", at + 1)
+    return out
+
+
+def test_page_aligned_kernels():
+    """The kernels marked T2R_PAGE start on a 4 KB page in the built code object."""
+    fns = _code_object_functions(abi.LIB_PATH)
+    for kernel in ("k_gemm_d", "k_attn_prep_h2", "k_rows_fin_quant"):
+        at = {n: a for n, (a, _) in fns.items() if kernel + "I" in n}
+        assert at and not any(a % 4096 for a in at.values()), at

@@ -1126,7 +1126,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void k_attn_prep_h(AttnArgs a) {
 // halves may hold a q and a k vector (odd H): each half stores what its vector writes. R: rows a
 // wave, every row's loads issued before the first row's steps.
 template <int HD, int R = 1>
-__global__ __launch_bounds__(64 * kPrepWaves) void k_attn_prep_h2(AttnArgs a, int rows) {
+__global__ T2R_PAGE __launch_bounds__(64 * kPrepWaves) void k_attn_prep_h2(AttnArgs a, int rows) {
   constexpr int NV = HD / 32;
   constexpr bool CONTIG = HD == 128;
   static_assert(NV == 2 || NV == 4, "head dims 64 and 128");

@@ -386,7 +386,7 @@ T2R_DEV void gemm_d_epilogue_vec(const GemmArgs& a, const v16i_t (&acc)[2][2], i
 
 // BM: tile rows (128: four waves, 2 x 2; 256: eight waves, 4 x 2), always 128 columns.
 template <int EPI, bool SPLIT, int BKD, int NST, int BM = kGT>
-__global__ __launch_bounds__(2 * BM, (BKD == 64 && NST == 3) ? 3 : 1) void k_gemm_d(GemmArgs a, int ntile, int nz) {
+__global__ T2R_PAGE __launch_bounds__(2 * BM, (BKD == 64 && NST == 3) ? 3 : 1) void k_gemm_d(GemmArgs a, int ntile, int nz) {
   constexpr int CPR = BKD / 16;                   // 16-byte chunks per row per slab
   constexpr int NWAVE = 2 * BM / 64;
   constexpr int NA = BM * CPR / 64;               // DMA instructions (1 KB each) of A per slab; B: 2 CPR

@@ -105,7 +105,7 @@ struct FinArgs {
 };
 
 template <int NCB>
-__global__ __launch_bounds__(kGemvThreads) void k_rows_fin_quant(GemvArgs a, FinArgs f) {
+__global__ T2R_PAGE __launch_bounds__(kGemvThreads) void k_rows_fin_quant(GemvArgs a, FinArgs f) {
   __shared__ __align__(16) int8_t xq_lds[1024 * NCB];
   __shared__ __align__(16) float xf_lds[1024 * NCB + 128];
   __shared__ __align__(16) float tab_lds[kSfuWords];
