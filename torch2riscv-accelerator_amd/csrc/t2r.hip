@@ -679,8 +679,8 @@ AttnArgs layer_attn_args(Model* m, int l, const int32_t* pos, int mode) {
   at.tab = sfu_table_ptr();
   at.qsum = d.attn_qsum;
   at.status = m->status;
-  // batch-1 decode over caches of more than one pass: each head's keys over 4 workgroups (k_attn_dec's
-  // SPLIT form), all of them resident at once (checked at creation)
+  // batch-1 decode at head dim 128 over caches of more than 512 rows: each head's keys over 4 workgroups
+  // (k_attn_dec's SPLIT form), all of them resident at once (checked at creation)
   if (mode == RUN_DECODE && m->nsplit > 1) {
     at.nsplit = m->nsplit;
     at.sp_s = m->sp_s; at.sp_o = m->sp_o; at.sp_acc = m->sp_acc; at.sp_sync = m->sp_sync;
@@ -1172,7 +1172,7 @@ int t2r_attn_prefill(const float* q, const int8_t* kc, const int8_t* vc, const i
   a.att = att; a.att_stride = (long long)H * hd;
   a.qsum = flags & T2R_ATTN_QSUM;
   a.ch_sk = ch_sk; a.ch_av = ch_av;
-  a.tab = sfu_table_ptr();                       // the multi-row kernel (k_attn_pre) where it takes the shape
+  a.tab = sfu_table_ptr();                       // the multi-row kernels where they take the shape
   return attn_launch(ATTN_ONLY, a, M, S(stream));
 }
 

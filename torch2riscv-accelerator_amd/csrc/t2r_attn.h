@@ -109,10 +109,11 @@ T2R_DEV void wave_mem_done() {
 }
 
 // A bounded wait for *p to reach want (modulo 2^32) at device scope (one lane polls); on running out
-// it sets bit 1 of *status and returns, so every workgroup reaches its end whatever happens. What the
-// caller reads after it from other workgroups it reads by agent-scope atomic loads, which no cache of this
-// XCD answers, so the wait needs no agent-scope acquire: that would drop the L2's K / V lines as well (C3's
-// decode step at 2000 positions 802 -> 794 us without it).
+// it sets bit 1 of *status and returns, so every workgroup reaches its end whatever happens. It acquires at
+// workgroup scope only (an agent-scope acquire drops the L2's K / V lines as well: C3's nine steps from 2032
+// positions 7431 -> 7529 us with one), so it makes no plain load of another workgroup's data safe. After it
+// such data is read by agent-scope atomic loads alone: on gfx950 no cache of this XCD answers them, and they
+// are issued once the poll's value is back.
 T2R_DEV void split_wait(uint32_t* p, uint32_t want, int32_t* status) {
   for (int it = 0; it < (1 << 20); ++it) {
     if ((int32_t)(__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - want) >= 0) {
@@ -466,8 +467,9 @@ T2R_DEV int slot_group_sum(int v) {
 // writes the output and clears the sums and its counter for the next launch. SPLIT 2 (no HF
 // options): each split stores its own int32 sums (splits past the passes store zeros) and the next
 // linear's prologue adds the four and scales them (F(f32(sum) a_v), the output's own formula).
-// A KV head's query heads run on one XCD (xcd_col) and the ordered sum's values are read 32 ahead: C4's decode
-// step at 100 / 600 / 2000 / 6100 positions 502 / 518 / 601 / 844 us before both, 500 / 510 / 568 / 751 after.
+// A KV head's query heads run on one XCD (xcd_col) and the ordered sum's values are read two sets of 16 ahead
+// (ordered_sum_long): C4's decode step at 100 / 600 / 2000 / 6100 positions 502 / 518 / 601 / 844 us before both,
+// 500 / 510 / 568 / 751 after.
 template <int NCH, bool OPT = false, int SPLIT = 0>   // 16-byte chunks per head row: hd = 16 NCH; OPT: the HF options
 __global__ __launch_bounds__(kAttnThreads) void k_attn_dec(AttnArgs a) {
   constexpr int HD = 16 * NCH;
@@ -2120,11 +2122,12 @@ __global__ __launch_bounds__(kApThreads, (ApCfg<HD, TW>::MINB)) void k_attn_pw(A
 //     k_attn_pw;
 //  3. e again, p = to_i8(...) packed as the MFMA A operand, P.V, as in k_attn_pw.
 // K and V tiles come by LDS DMA into slots of the wave's own, each refilled as soon as its operands
-// are in registers, and a wave's tiles need no registers beyond the one at hand, so two workgroups
-// share a CU: one's chains and barriers overlap the other's EXPs. Bound by the VALU (two EXPs a key,
-// about 45 steps without qsum). 1001 rows of 32 heads at head dim 64 from position 2500: 127 us, against
-// 1190 in k_attn's workgroup per (head, row); with qsum (one EXP a key, no chains) 777 rows of 16 heads at
-// head dim 128 from position 500: 27.6 us, against 74.4 in k_attn_pre.
+// are in registers, and a wave keeps no tile but the one at hand: 128 registers at most (at head dim 128 seven
+// without the options and nine with them are spilled), so two workgroups share a CU: one's chains and barriers
+// overlap the other's EXPs. Bound by the VALU (two EXPs a key, about 45 steps without qsum). 1001 rows of 32
+// heads at head dim 64 from position 2500: 127 us, against 1190 in k_attn's workgroup per (head, row); with qsum
+// (one EXP a key, no chains) 777 rows of 16 heads at head dim 128 from position 500: 27.6 us, against 74.4 in
+// k_attn_pre. For few rows the others are faster (ps_takes).
 template <int HD> struct AsCfg { static constexpr int RING = HD == 64 ? 2 : 1; };
 template <int HD> constexpr size_t as_lds() {             // K slots, then the exp chunk / the V slots
   constexpr size_t k = (size_t)kApWaves * AsCfg<HD>::RING * 32 * HD;
@@ -2487,8 +2490,8 @@ inline size_t attn_dec_lds_bytes(int S, int D) { return ((size_t)D * osum_stride
 
 // ------------------------------------------------------------------ grouped decode attention
 // Decode attention of the G <= 4 query heads that share a KV head, split over G / GW workgroups per
-// (row, KV head g), each taking GW of the group's query heads (2 for four-head groups, else 1): the
-// numerics are k_attn_dec's step for step, the work is split differently.
+// (row, KV head g), each taking GW of the group's query heads (2 for four-head groups of many rows, else 1:
+// attn_launch has the line): the numerics are k_attn_dec's step for step, the work is split differently.
 //  - Vector jobs, one per wave: the KV head (k: QK-norm, RoPE, int8; v: int8; the cache row) and
 //    the workgroup's GW query heads (QK-norm, RoPE, quant_act). Every workgroup of the KV head forms
 //    its new row; split 0 is the only one that writes it to the cache.
