@@ -1701,10 +1701,10 @@ inline size_t attn_pre_lds_bytes(int S, int HDP) {
 //  - the waves' int32 sums added by LDS integer atomics (exact in any order) and scaled.
 // TW 8 (up to 2048 positions) keeps 8 tiles a wave: 128 score registers, one workgroup per CU, a
 // four-tile K ring, two exp-chunk buffers. TW 2 (512 positions, head dim 64) leaves room for two
-// workgroups a CU. Bound by the VALU steps of a key (about 40, 14 of them EXP). 512 rows of 32 heads at
-// head dim 64 attending to 1520..2031 positions: 36.6 us, against 104 in k_attn_pre's 16-row blocks
-// (which read K and V twice as often and run one thread per key chain) and 44.3 streamed (k_attn_ps);
-// at 512..1023 positions 22.8, 61 and 25.6 us.
+// workgroups a CU. Bound by the VALU steps of a key (about 40, 14 of them EXP: half of the time if issued
+// evenly) and the chunks' barriers. 512 rows of 32 heads at head dim 64 attending to 1520..2031 positions:
+// 36.6 us, against 104 in k_attn_pre's 16-row blocks (which read K and V twice as often and run one thread per
+// key chain) and 44.3 streamed (k_attn_ps); at 512..1023 positions 22.8, 61 and 25.6 us.
 constexpr int kApRows = 32, kApThreads = 512, kApWaves = kApThreads / 64;
 constexpr int kApStage = 256 + 16;                       // float stride of a row of a 256-key chunk
 // TW: the tiles a wave keeps (TW 256 positions)
@@ -2124,10 +2124,11 @@ __global__ __launch_bounds__(kApThreads, (ApCfg<HD, TW>::MINB)) void k_attn_pw(A
 // K and V tiles come by LDS DMA into slots of the wave's own, each refilled as soon as its operands
 // are in registers, and a wave keeps no tile but the one at hand: 128 registers at most (at head dim 128 seven
 // without the options and nine with them are spilled), so two workgroups share a CU: one's chains and barriers
-// overlap the other's EXPs. Bound by the VALU (two EXPs a key, about 45 steps without qsum). 1001 rows of 32
-// heads at head dim 64 from position 2500: 127 us, against 1190 in k_attn's workgroup per (head, row); with qsum
-// (one EXP a key, no chains) 777 rows of 16 heads at head dim 128 from position 500: 27.6 us, against 74.4 in
-// k_attn_pre. For few rows the others are faster (ps_takes).
+// overlap the other's EXPs. Without qsum bound by the VALU (two EXPs a key, about 45 steps): 1001 rows of 32 heads
+// at head dim 64 from position 2500 127 us (72.7M VALU instructions, 118 us if spread evenly), against 1190 in
+// k_attn's workgroup per (head, row). With qsum (one EXP a key, no chains) 777 rows of 16 heads at head dim 128
+// from position 500: 27.6 us, against 74.4 in k_attn_pre; 11 us of it VALU issue, the rest waits on the one K slot
+// a wave. For few rows the others are faster (ps_takes).
 template <int HD> struct AsCfg { static constexpr int RING = HD == 64 ? 2 : 1; };
 template <int HD> constexpr size_t as_lds() {             // K slots, then the exp chunk / the V slots
   constexpr size_t k = (size_t)kApWaves * AsCfg<HD>::RING * 32 * HD;

@@ -187,7 +187,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm(const float* x, const float* g,
 // k_rmsnorm for rows of whole 16-byte groups (n % 16 == 0, 16-byte aligned rows and gains, n <= 1024 NCB):
 // x and the gain in registers by 16-byte loads requested together, the squares lane-major in LDS for the
 // one ordered chain (the GEMV prologue's form), 16-byte stores. Bound by that chain and three round trips:
-// one row of 2048 values 3.1 us, against 5.7 in k_rmsnorm; 1001 rows 15.0 in k_rmsnorm.
+// one row of 2048 values 3.1 us, against 5.7 in k_rmsnorm; 1001 rows 7.6, against 15.0.
 template <int NCB>
 __global__ __launch_bounds__(kGemvThreads) void k_rmsnorm_rows(GemvArgs a, float* out) {
   constexpr int NX = NCB;                          // float4 a thread
@@ -795,7 +795,7 @@ __global__ __launch_bounds__(256) void k_moe_down(MoeDownArgs m) {
 // requested together) and keeps their maximum (NaN winning, half an instruction a value) with the first
 // pass that raised it; then only the threads that hold the row's maximum look at that pass's values
 // again for the first index. 128256 values: 155.6 us as a 64-bit (value, index) key per value on 256
-// threads with one 4-byte load in flight each, 7.6 us this way.
+// threads with one 4-byte load in flight each, 7.8 us this way.
 constexpr int kArgmaxThreads = 1024;
 __global__ __launch_bounds__(kArgmaxThreads) void k_argmax(const float* x, int n, int32_t* idx) {
   typedef float v4u_t __attribute__((ext_vector_type(4), aligned(4)));   // (a row may start at any float)
